@@ -28,6 +28,7 @@
 #include "a8w8_common.h"
 
 #include <atomic>
+#include <cmath>
 
 // The scaled output is two fp32 multiplications and one rounding to 16 bits, each rounded on its
 // own as in the reference's torch path.
@@ -69,6 +70,19 @@ struct OptionalStage<false, BYTES> {
     static __device__ __forceinline__ char* get() { return nullptr; }
 };
 
+// The kernel's own arguments read again from where the launch put them.  The tile code inside a loop gets them so: left to
+// the compiler every argument that the loop needs again stays in scalar registers over the tile (70 of them spilled,
+// and with them 27 vector registers of the 256x256 tile).
+struct Kernargs { A8W8Args p; MoeArgs moe; };
+__device__ __forceinline__ Kernargs kernargs() {
+    typedef const __attribute__((address_space(4))) char* const_ptr_t;
+    const_ptr_t k = (const_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    Kernargs r;
+    __builtin_memcpy(&r, k, sizeof(r));
+    return r;
+}
+
 // SPLIT: the workgroups of the grid are units, kparts per tile, each the tile's product over its own range
 // of K (k_chunk bytes per row, a multiple of the slab; the last part takes the rest).  A unit that is done
 // counts itself arrived at the tile's counter.  If it is the last to arrive and finds every other unit's
@@ -80,12 +94,15 @@ struct OptionalStage<false, BYTES> {
 // the unsplit kernel's bit for bit.  The unit that adds up sets the counter back to zero: the counters are
 // zero whenever no call is in flight.
 // MOE: the mixture-of-experts form for many routed rows per expert (flashnn/triton_kernels/fused_moe_a8w8.py:37-173).
-// The M dimension is the list of sorted routed rows (moe.EM of them, padded per expert to blocks of moe.block_m, a
-// multiple of BM): tile row r multiplies activation row sorted_ids[r] / top_k with the weight matrix of the
-// expert its block belongs to, and the result goes to output row sorted_ids[r], times the routing weight on
-// request.  Tiles beyond the rows in use return at once; padding rows read activation row 0 and store nothing.
-template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2, bool SPLIT = false, bool MOE = false>
-__global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Args p, const MoeArgs moe) {
+// The M dimension is the list of sorted routed rows (moe.EM of them, padded per expert to blocks of moe.block_m): tile
+// row r multiplies activation row sorted_ids[r] / top_k with the weight matrix of the expert its block belongs to, and
+// the result goes to output row sorted_ids[r], times the routing weight on request.  A tile is a part of one block or
+// a few blocks of one expert (MoeTiles); padding rows read activation row 0 and store nothing.
+//
+// One tile: rows m0 .. of the tile (MOE: sorted rows, those from row_end on are padding), columns n0 ..; part kpart of K.
+template <int BM, int BN, int MODE, bool PAIR, int WGM, bool SPLIT, bool MOE>
+__device__ __forceinline__ void ring_tile(const A8W8Args& p, const MoeArgs& moe, const int t, const int kpart, const int m0,
+                                          const int n0, const int row_end, const int expert, const int tid) {
     static_assert(!MOE || (!SPLIT && MODE != OUT_I32), "the gathered form has no split and no raw output");
     // WGM x 2 waves.  Only WGM = 2 (one wave per SIMD) is instantiated: with WGM = 4 the two waves of a SIMD
     // meet at the same barrier every slab and never filled each other's gaps (256x192: 81.6 us with four
@@ -124,40 +141,19 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
     float* const sc_row = (float*)sb2;
     float* const sc_col = sc_row + BM;
 
-    const int xcd = blockIdx.x & 7;
-    const int unit = xcd * p.tiles_per_xcd + (blockIdx.x >> 3);   // (tiles_per_xcd counts units where SPLIT)
-    if ((blockIdx.x >> 3) >= p.tiles_per_xcd || unit >= p.tiles_m * p.tiles_n * (SPLIT ? p.kparts : 1)) return;
-    // the units of a tile are neighbours in this numbering: they run on one XCD, at about the same time
-    const int t = SPLIT ? unit / p.kparts : unit;
-    const int kpart = SPLIT ? unit - t * p.kparts : 0;
     const int8_t* const pa = SPLIT ? p.a + (int64_t)kpart * p.k_chunk : p.a;
-    const int8_t* pb = SPLIT ? p.b + (int64_t)kpart * p.k_chunk : p.b;
+    const int8_t* const pb = MOE ? p.b + (int64_t)expert * moe.stride_be : SPLIT ? p.b + (int64_t)kpart * p.k_chunk : p.b;
     // (the last part takes what the others leave: a few slabs more, so that it arrives last as a rule)
     const int Kl = SPLIT ? (kpart == p.kparts - 1 ? p.K - kpart * p.k_chunk : p.k_chunk) : p.K;
-    // tiles are numbered in groups of GN tile columns, the column fastest within a group: the 32 workgroups
-    // an XCD runs at a time then cover 32 / GN tile rows x GN tile columns whatever M is, and fetch
-    // (32 / GN) * BM + GN * BN operand rows per slab into its L2 instead of tiles_m*BM + BN.  GN = 8 for the tiles
-    // of 192 and 256 columns, 4 for the narrower ones (measured, see the launchers).
-    const int GN = p.gn;
-    const int grp = t / (GN * p.tiles_m);
-    const int rem = t - grp * (GN * p.tiles_m);
-    const int gw = min(GN, p.tiles_n - grp * GN);
-    const int tile_n = grp * GN + rem % gw;
-    const int tile_m = rem / gw;
-    const int m0 = tile_m * BM;
-    const int n0 = tile_n * BN;
-    int expert = 0;
-    if constexpr (MOE) {
-        if (m0 >= moe.ntpp[0]) return;
-        expert = moe.expert_ids[m0 / moe.block_m];
-        pb += (int64_t)expert * moe.stride_be;
-    }
     // the routed row of tile row r (MOE), and the activation row it reads: padding rows read row 0
-    auto routed = [&](int r) -> int { return moe.sorted_ids[min(m0 + r, moe.EM - 1)]; };
+    auto routed = [&](int r) -> int {
+        const int tok = moe.sorted_ids[min(m0 + r, row_end - 1)];
+        return m0 + r < row_end ? tok : moe.num_valid;
+    };
     auto act_row = [&](int tok) -> int { return tok < moe.num_valid ? tok / moe.top_k : 0; };
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WGM;
     const int wn = wave / WGM;
 
@@ -170,7 +166,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
     if constexpr (MODE != OUT_I32) {
 #pragma unroll
         for (int q = 0; q < NSC; ++q) {
-            const int e = threadIdx.x + q * NT;
+            const int e = tid + q * NT;
             const bool is_row = e < BM;
             int64_t idx = is_row ? min(m0 + e, p.M - 1) : min(n0 + min(e - BM, BN - 1), p.N - 1);
             if constexpr (MOE) idx = is_row ? act_row(routed(e)) : idx + (int64_t)expert * moe.stride_scale_be;
@@ -200,7 +196,13 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
     // The address of a copy is a scalar base (matrix + slab) plus the lane's 32-bit row offset, which is the
     // form the copy instruction takes directly; the base is passed through readfirstlane so that it is not
     // folded into per-lane 64-bit pointers that need vector adds before every copy.
+    // Where weight rows lie a multiple of 4 KiB apart, the pieces of all rows of all tiles that are at the same slab come
+    // from the same few memory channels: tile column c then starts p.rot * c slabs into K and goes round (the last slab,
+    // which may be partial, stays the last).  Integer sums do not depend on the order.
+    const int whole = (Kl + BK - 1) / BK - 1;
+    const int rot = MOE ? (n0 / BN * p.rot) % whole : 0;
     auto slab_base = [&](const int8_t* m, int kt) -> const char* {
+        if (MOE && kt < whole) kt = kt + rot - (kt + rot >= whole ? whole : 0);
         const uint64_t v = (uint64_t)m + (uint64_t)((int64_t)kt * BK);
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
@@ -484,7 +486,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         // The tile's counter holds arrivals in its low half and completed slots in its high half.
         int* const word = (int*)sb2 + BM + BN;      // behind the scales' place in the third b-stage
         __syncthreads();                    // every wave has left the main loop: the stages are free
-        if (threadIdx.x == 0)
+        if (tid == 0)
             *word = __hip_atomic_fetch_add(p.ws_count + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         const int seen = *word;
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
             for (int i = 0; i < FN; ++i)
 #pragma unroll
                 for (int j = 0; j < FM; ++j)
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[i][j]), mine, threadIdx.x * 16,
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[i][j]), mine, tid * 16,
                                                            (i * FM + j) * (NT * 16), 16 /* sc1 */);
             // Every wave waits here until all of its slot stores have been acknowledged (vmcnt counts a
             // store until the memory side has taken it); only behind the barrier that follows does one
@@ -510,7 +512,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
             __builtin_amdgcn_s_waitcnt(0x0070);
             asm volatile("" ::: "memory");
             __syncthreads();
-            if (threadIdx.x == 0)
+            if (tid == 0)
                 *word = __hip_atomic_fetch_add(p.ws_count + t, 0x10000, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             // whoever completes the last of all kparts slots adds up the others; otherwise this unit is done
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         asm volatile("" ::: "memory");
         for (int q = 0; q < p.kparts; ++q) {
             if (q == kpart) continue;
-            const u64* const theirs = slots + (int64_t)q * (BM * BN / 2) + 2 * threadIdx.x;
+            const u64* const theirs = slots + (int64_t)q * (BM * BN / 2) + 2 * tid;
 #pragma unroll
             for (int i = 0; i < FN; ++i)
 #pragma unroll
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
                     acc[i][j] += v4i{(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
                 }
         }
-        if (threadIdx.x == 0) __hip_atomic_store(p.ws_count + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) __hip_atomic_store(p.ws_count + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
     // ---- epilogue ----
@@ -571,13 +573,16 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         // the three instructions of a fragment row the wave's whole 192-byte (WTN * 2) piece of them.  No
         // LDS transposition, no barrier between the waves.
         static_assert(FN % 2 == 0, "weight fragments are stored in pairs");
+        const Kernargs again = MOE ? kernargs() : Kernargs{p, moe};
+        const A8W8Args& p = again.p;
+        const MoeArgs& moe = again.moe;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0x0070);   // all copies and LDS reads of this wave are done
         __builtin_amdgcn_s_barrier();         // ... and everybody else's: the stages are free
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int q = 0; q < NSC; ++q) {
-            const int e = threadIdx.x + q * NT;
+            const int e = tid + q * NT;
             const bool is_row = e < BM;
             const int dt = is_row ? p.arow_dtype : p.acol_dtype;
             const float v = dt == FNN_F32 ? __builtin_bit_cast(float, sc_raw[q])
@@ -589,7 +594,7 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         int* const sc_tok = (int*)(sc_col + BN) + 4;
         float* const sc_wr = (float*)(sc_tok + BM);
         if constexpr (MOE) {
-            for (int e = threadIdx.x; e < BM; e += NT) {
+            for (int e = tid; e < BM; e += NT) {
                 const int tok = routed(e);
                 sc_tok[e] = tok;
                 sc_wr[e] = moe.mul_w && tok < moe.num_valid ? load_as_f32(moe.topk_w, tok, moe.topk_w_dtype) : 1.f;
@@ -717,6 +722,52 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         if (inside && !MOE) store_full(std::false_type{});
         else if (cols_inside) store_full(std::true_type{});
         else store_rows();
+    }
+}
+
+template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2, bool SPLIT = false, bool MOE = false>
+__global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Args p, const MoeArgs moe) {
+    const int xcd = blockIdx.x & 7;
+    // tiles are numbered in groups of gn tile columns, the column fastest within a group: the 32 workgroups
+    // an XCD runs at a time then cover 32 / gn tile rows x gn tile columns whatever M is, and fetch
+    // (32 / gn) * BM + gn * BN operand rows per slab into its L2 instead of tiles_m*BM + BN.  gn = 8 for the tiles
+    // of 192 and 256 columns, 4 for the narrower ones (measured, see the launchers).
+    auto place = [&](int t, int tiles_m, int& tile_m, int& tile_n) {
+        const int grp = t / (p.gn * tiles_m);
+        const int rem = t - grp * (p.gn * tiles_m);
+        const int gw = min(p.gn, p.tiles_n - grp * p.gn);
+        tile_n = grp * p.gn + rem % gw;
+        tile_m = rem / gw;
+    };
+    int tile_m, tile_n;
+    if constexpr (MOE) {
+        // The number of tiles is known on the device only.  The grid is the host's estimate of it (p.tiles_per_xcd
+        // workgroups per XCD); where there are more, workgroups take a second tile.
+        int slot = blockIdx.x >> 3;
+        for (;;) {
+            const MoeTiles<BM> map(moe);
+            const int tiles = map.tiles * p.tiles_n, per_xcd = (tiles + 7) / 8;
+            const int t = xcd * per_xcd + slot;
+            if (slot >= per_xcd || t >= tiles) return;
+            place(t, map.tiles, tile_m, tile_n);
+            int m0, rows, expert;
+            map.find(tile_m, m0, rows, expert);
+            const Kernargs k = kernargs();
+            int tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));          // (so that what a lane derives from its number is not kept either)
+            ring_tile<BM, BN, MODE, PAIR, WGM, SPLIT, MOE>(k.p, k.moe, t, 0, m0, tile_n * BN, m0 + rows, expert, tid);
+            slot += p.tiles_per_xcd;
+            __builtin_amdgcn_s_waitcnt(0x0070);     // this tile's stores are out, and nobody reads its LDS any more
+            __syncthreads();
+        }
+    } else {
+        const int unit = xcd * p.tiles_per_xcd + (blockIdx.x >> 3);   // (tiles_per_xcd counts units where SPLIT)
+        if ((blockIdx.x >> 3) >= p.tiles_per_xcd || unit >= p.tiles_m * p.tiles_n * (SPLIT ? p.kparts : 1)) return;
+        // the units of a tile are neighbours in this numbering: they run on one XCD, at about the same time
+        const int t = SPLIT ? unit / p.kparts : unit;
+        place(t, p.tiles_m, tile_m, tile_n);
+        ring_tile<BM, BN, MODE, PAIR, WGM, SPLIT, MOE>(p, moe, t, SPLIT ? unit - t * p.kparts : 0, tile_m * BM, tile_n * BN,
+                                                       p.M, 0, threadIdx.x);
     }
 }
 
@@ -1076,40 +1127,68 @@ static void dispatch(A8W8Args& p, hipStream_t st, int force_bm, int force_bn, in
         }
 }
 
-// Mixture of experts with many routed rows per expert: the MFMA tiles over the sorted rows.  A tile must lie
-// within one expert's rows, so its height divides block_m.  Returns false where this form does not apply (the
-// few-row kernels then take the call).
+// Mixture of experts with many routed rows per expert: the MFMA tiles over the sorted rows.  Returns false where this
+// form does not apply (the few-row kernels then take the call).
 template <int BM, int BN, int MODE, bool PAIR = false>
 static void launch_mfma_moe(A8W8Args& p, const MoeArgs& q, hipStream_t st) {
-    p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
-    p.tiles_per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
+    p.tiles_per_xcd = (int)((moe_tiles_estimate(q, BM) * p.tiles_n + 7) / 8);   // workgroups per XCD
     p.gn = 4;
-    note_kernel("gemm_a8w8_ring_kernel(moe)", BM, BN, 4);
+    // (same box, microseconds, 8 experts, rotation 0 / 1 / 11 - N = 8192 K = 4096: 24 rows per expert, 64-row tiles 71.5 /
+    // 61.5 / 56.2; 100 rows, 128-row tiles 80 / 70.5 / 64.5; 250 rows, 256-row tiles 127 / 121 / 124, 1000 rows 296 / 297 /
+    // 305.  N = 8192 K = 8192: 113 / 102 / 103; 136 / 109 / 118; 210 / 202 / 209; 501 / 497 / 522.  With more than one tile
+    // row per expert the wide step takes tiles that share activation rows too far apart.  K = 7168, 14336: no difference)
+    p.rot = p.ldb % 4096 != 0 ? 0 : BM == 64 ? 11 : 1;
+    note_kernel(q.block_m < BM ? "gemm_a8w8_ring_kernel(moe, blocks together)" : "gemm_a8w8_ring_kernel(moe)", BM, BN, 4);
     gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, 2, false, true><<<dim3(p.tiles_per_xcd * 8), dim3(256), 0, st>>>(p, q);
 }
 
+// Tile heights that the block size allows: the tile is a part of a block, or whole blocks make up the tile.
+static bool moe_tile_fits(const MoeArgs& q, int bm) { return q.block_m >= 16 && (q.block_m % bm == 0 || bm % q.block_m == 0); }
+
+// The height of the tiles.  Blocks of a multiple of 128 rows keep tiles of at least 128, of 256 rows those of 256 (what the
+// caller sorted for).  Else by the mean number of routed rows per expert (estimated, moe_experts_estimate), where the
+// tiles fill the chip; with fewer than one round of the taller tiles, 64 rows.  Measured over
+// E x N x K = 8 x 28672 x 4096 | 16 x 12288 x 4096 | 8 x 4096 x 14336 | 64 x 2816 x 2048, tiles of 64 / 128 / 256 rows,
+// microseconds: 50 rows per expert 192 / 197 / 278 | 183 / 193 / 234 | 106 / 99 / 155 | 90 / 92 / 127 (56 rows); 75 rows 247 /
+// 205 / 282 | 215 / 198 / 238 | 128 / 105 / 158; 100 rows 261 / 212 / 283 | 251 / 237 / 237 (128 rows) | 132 / 113 / 160 |
+// 114 / 98 / 128; 150 rows 314 / 303 / 291 | - | 169 / 150 / 164; 256 rows 429 / 366 / 361 | 375 / 327 / 322 | 232 / 221 /
+// 181 | 170 / 155 / 136 (192 rows); 1024 rows 1375 / 1128 / 999 | - | 710 / 557 / 509 | 274 / 261 / 259 (384 rows).
+static int moe_tile_rows(const A8W8Args& p, const MoeArgs& q) {
+    const int least = q.block_m % 256 == 0 ? 256 : q.block_m % 128 == 0 ? 128 : 64;
+    const double mean = (double)q.num_valid / (double)moe_experts_estimate(q);
+    int bm = mean <= 56 ? 64 : mean < 144 ? 128 : 256;
+    while (bm > least && (!moe_tile_fits(q, bm) || moe_tiles_estimate(q, bm) * ((p.N + bm - 1) / bm) < 256)) bm /= 2;
+    return bm > least ? bm : least;
+}
+
 template <int MODE>
-static bool launch_moe_tiled_t(A8W8Args& p, const MoeArgs& q, hipStream_t st) {
-    if (q.block_m % 256 == 0) launch_mfma_moe<256, 256, MODE>(p, q, st);
-    else if (q.block_m % 128 == 0) launch_mfma_moe<128, 128, MODE, true>(p, q, st);
+static void launch_moe_tiled_t(A8W8Args& p, const MoeArgs& q, int bm, hipStream_t st) {
+    if (bm == 256) launch_mfma_moe<256, 256, MODE>(p, q, st);
+    else if (bm == 128) launch_mfma_moe<128, 128, MODE, true>(p, q, st);
     else launch_mfma_moe<64, 128, MODE>(p, q, st);
-    return true;
 }
 
 static bool launch_a8w8_moe_tiled(A8W8Args& p, const MoeArgs& q, int mode, hipStream_t st) {
     constexpr int64_t kLimit = (1LL << 31) - 1;
     const int64_t rows = (q.num_valid + q.top_k - 1) / q.top_k;          // activation rows
-    const bool ok = q.block_m % 64 == 0 && q.EM % q.block_m == 0 && p.K % 32 == 0 && p.K >= 1024 &&
+    const int bm = q.block_m >= 16 && q.EM % q.block_m == 0 ? moe_tile_rows(p, q) : 0;
+    const bool ok = bm > 0 && moe_tile_fits(q, bm) && p.K % 32 == 0 && p.K >= 1024 &&
                     p.lda % 16 == 0 && p.ldb % 16 == 0 && q.stride_be % 16 == 0 && ((uintptr_t)p.a % 16) == 0 &&
                     ((uintptr_t)p.b % 16) == 0 && ((uintptr_t)p.out % 16) == 0 && rows * p.lda <= kLimit &&
-                    (int64_t)p.N * p.ldb <= kLimit && (int64_t)(p.M / 64) * ((p.N + 127) / 128) <= kLimit;
-    // The few-row kernel reads an expert's weights once per 64 sorted rows.  Measured on 8 experts of
-    // 28672 x 4096, 2 per token, microseconds over S sorted rows in use: few-row kernel 100 + 0.18 S; tiles of
-    // 64 rows 110 + 0.14 S, of 128 rows 105 + 0.10 S, of 256 rows 57 + 0.092 S.  Blocks of 128 rows or more
-    // always take the tiles; blocks of 64 from about 512 routed rows on.
-    if (!ok || (q.block_m % 128 != 0 && q.num_valid < 512)) return false;
-    return mode == OUT_F16 ? launch_moe_tiled_t<OUT_F16>(p, q, st) : launch_moe_tiled_t<OUT_BF16>(p, q, st);
+                    (int64_t)p.N * p.ldb <= kLimit && moe_tiles_estimate(q, 64) * ((p.N + 127) / 128) <= kLimit;
+    if (!ok) return false;
+    // Few tiles of long rows leave most CUs without one: the few-row kernel, whose workgroups own 16 to 64 channels, is ahead
+    // (8 experts, N = 4096 K = 14336, blocks of 16, few-row kernel / 64-row tiles, us: 1 token 41 / 58, 2 tokens 51 / 63, 3
+    // tokens 62 / 67, 4 tokens 80 / 71, 16 tokens 99 / 87, 64 tokens 142 / 88; N = 2816 K = 2048, 64 experts, 6 per token: 1
+    // token 24 / 20, 64 tokens 159 / 79; N = 28672 K = 4096: 1 token 69 / 49, 8 tokens 150 / 160, 16 tokens 165 / 168, 64
+    // tokens 229 / 175; N = 12288 K = 4096, 16 experts: 1 token 35 / 26, 64 tokens 151 / 148).
+    const double experts = (double)moe_experts_estimate(q);
+    const double reached = experts * (1.0 - pow(1.0 - 1.0 / experts, (double)q.num_valid));
+    if (bm == 64 && q.block_m < 64 && p.K >= 8192 && reached * ((p.N + 127) / 128) < 150) return false;
+    if (mode == OUT_F16) launch_moe_tiled_t<OUT_F16>(p, q, bm, st);
+    else launch_moe_tiled_t<OUT_BF16>(p, q, bm, st);
+    return true;
 }
 
 static int check_args(const char* fn, const void* out, const void* a, const void* b, int64_t M,

@@ -21,4 +21,86 @@ struct MoeArgs {
     int64_t stride_scale_n, stride_scale_k, stride_zp_n, stride_zp_k;
 };
 
+// The tiles of BM sorted rows that a tiled kernel cuts the routed rows into.  Blocks of BM rows and more are cut into
+// whole tiles.  Smaller blocks are put together: a tile is up to BM / block_m consecutive blocks of one expert, so the
+// height of the tile - what decides how often an expert's weights are read, and how many operand bytes a CU takes in per
+// output - does not hang on the block size that the caller sorted for.  Where an expert's blocks end, and so how many tiles
+// there are, is read from expert_ids by every wave for itself: 64 blocks per step, four steps' loads in flight (256
+// blocks: one L2 latency, about 1 us before a tile of 40 to 60 us).
+template <int BM>
+struct MoeTiles {
+    const MoeArgs& q;
+    int blocks, tiles;       // blocks in use and tiles that they make
+
+    __device__ __forceinline__ explicit MoeTiles(const MoeArgs& args) : q(args) {
+        const int used = min(q.ntpp[0], q.EM);
+        blocks = __builtin_amdgcn_readfirstlane((used + q.block_m - 1) / q.block_m);
+        tiles = q.block_m >= BM ? blocks * (q.block_m / BM) : scan(-1);
+    }
+
+    // the number of tiles (want < 0), or the first block of tile `want`
+    __device__ __forceinline__ int scan(int want) const {
+        const int lane = threadIdx.x & 63, r = BM / q.block_m;
+        int count = 0, last_expert = 0, run = 0;        // run: first block of the expert's blocks that are being walked
+        for (int base = 0; base < blocks; base += 256) {
+            int e[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[c] = q.expert_ids[min(base + 64 * c + lane, blocks - 1)];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int first = base + 64 * c, blk = first + lane;
+                if (first >= blocks) break;
+                const int before = __shfl_up(e[c], 1, 64);
+                const bool starts = blk < blocks && (blk == 0 || e[c] != (lane == 0 ? last_expert : before));
+                const uint64_t runs = __ballot(starts);
+                const uint64_t here = runs & (~0ull >> (63 - lane));
+                const int mine = here ? first + 63 - __clzll(here) : run;
+                const uint64_t heads = __ballot(blk < blocks && (blk - mine) % r == 0);
+                const int n = __popcll(heads);
+                if (want >= 0 && want < count + n) {
+                    const bool hit = (heads >> lane & 1) && __popcll(heads & ((1ull << lane) - 1)) == want - count;
+                    return __builtin_amdgcn_readfirstlane(first + __ffsll((unsigned long long)__ballot(hit)) - 1);
+                }
+                count += n;
+                last_expert = __builtin_amdgcn_readlane(e[c], 63);
+                if (runs) run = first + 63 - __clzll(runs);
+            }
+        }
+        return count;
+    }
+
+    // first sorted row of a tile, how many of its rows belong to it, and their expert
+    __device__ __forceinline__ void find(int tile, int& m0, int& rows, int& expert) const {
+        if (q.block_m >= BM) {
+            m0 = tile * BM;
+            rows = BM;
+            expert = q.expert_ids[m0 / q.block_m];
+        } else {
+            const int lane = threadIdx.x & 63, r = BM / q.block_m, b = scan(tile);
+            const int e = q.expert_ids[min(b + lane, blocks - 1)];
+            expert = __builtin_amdgcn_readfirstlane(e);
+            const uint64_t same = __ballot(lane < r && b + lane < blocks && e == expert);
+            m0 = b * q.block_m;
+            rows = (__ffsll((unsigned long long)~same) - 1) * q.block_m;
+        }
+    }
+};
+
+// What the host can say about the routing without reading it: the sorted list holds every routed row and up to
+// block_m - 1 padding rows per expert, which gives the number of experts it was made for.  An estimate (a caller may cut
+// its list): used for grid sizes and prices only.
+inline int64_t moe_experts_estimate(const MoeArgs& q) {
+    const int64_t blocks = q.EM / q.block_m, pad = (int64_t)q.EM - q.num_valid;
+    if (pad <= 0 || q.block_m < 2) return 1;
+    const int64_t e = (pad + q.block_m - 2) / (q.block_m - 1);
+    return e < blocks ? e : (blocks > 0 ? blocks : 1);
+}
+// ... and so the number of tiles of bm rows
+inline int64_t moe_tiles_estimate(const MoeArgs& q, int bm) {
+    const int64_t blocks = q.EM / q.block_m;
+    if (q.block_m >= bm) return blocks * (q.block_m / bm);
+    const int64_t t = (q.num_valid + bm - 1) / bm + moe_experts_estimate(q);
+    return t < blocks ? t : blocks;
+}
+
 }  // namespace fnn

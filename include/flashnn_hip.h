@@ -343,11 +343,11 @@ int fnn_gemm_a8w8_i32_tiled(int32_t* acc, const void* a, const void* b, int64_t 
  * times topk_weights[t] when mul_routed_weight != 0; every product rounded to fp32, the result rounded
  * once to out_dtype (the reference always rounds to fp16, :162).  Rows of c that no valid sorted row names
  * are left untouched.  sorted_token_ids [EM], expert_ids and num_tokens_post_padded [1] are int32 device
- * arrays.  The weight-streaming kernel takes N % 16 == 0, K % 32 == 0, K >= 1024, block_m % 16 == 0,
- * EM % block_m == 0 and 16-byte aligned rows; anything else takes a slow guarded kernel.
- * Many routed rows per expert: with block_m a multiple of 128 (or of 64, from 512 routed rows on) and
- * K >= 1024 the call runs MFMA tiles over the sorted rows (tile height 64, 128 or 256 = the largest of those
- * that divides block_m) instead of streaming an expert's weights once per 64 rows; same arithmetic, same bits.
+ * arrays.  K >= 1024, K % 32 == 0, EM % block_m == 0, 16-byte aligned rows and block_m 16, 32, 64 or a multiple of 64:
+ * MFMA tiles of 64, 128 or 256 sorted rows.  A tile is a part of one block or, where blocks are smaller, several
+ * consecutive blocks of one expert, so block_m decides the padding and not the speed.  A few rows over few channels,
+ * and other multiples of 16, take a weight-streaming kernel (N % 16 == 0); anything else a slow guarded kernel.  The same
+ * arithmetic and the same bits everywhere.
  */
 int fnn_fused_moe_a8w8(void* c, const void* a, const void* b, const void* alpha_row,
                        const void* alpha_col, const void* topk_weights,

@@ -677,6 +677,49 @@ def test_fused_moe_a8w8_many_rows_bit_exact(shape, out_ty):
             assert (want == 3.0).any()
 
 
+@pytest.mark.parametrize("shape", [
+    # M, E, N, K, top_k, block, tile rows
+    (1000, 8, 12304, 1056, 2, 64, 256), (300, 8, 4096, 4096, 2, 16, 128), (45, 5, 1040, 1024, 3, 16, 64),
+    (700, 70, 2064, 1024, 6, 32, 128), (1, 4, 528, 1120, 1, 16, 64), (160, 1, 22032, 1024, 2, 64, 256)])
+def test_fused_moe_a8w8_blocks_put_together(shape):
+    """Blocks smaller than the tile: a tile is several blocks of one expert, and the result has the bits of the same
+    routing sorted in blocks of 256 rows (one block per tile) - with the experts' blocks in order, with the blocks
+    shuffled (runs of one block each, more tiles than the grid was sized for) and with a list cut in the middle."""
+    M, E, N, K, top_k, BM, tile_rows = shape
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randint(-128, 128, (M, K), dtype=torch.int8, generator=g).to(DEV)
+    b = torch.randint(-128, 128, (E, N, K), dtype=torch.int8, generator=g).to(DEV)
+    ar = (torch.rand(M, generator=g) * 0.05).half().to(DEV)
+    ac = (torch.rand(E, N, generator=g) * 0.05).to(DEV)
+    ids = torch.stack([torch.randperm(max(E, top_k), generator=g)[:top_k] % E for _ in range(M)])
+    w = torch.rand(M, top_k, generator=g).to(DEV)
+
+    def run(s, e, used, block):
+        c = torch.full((M, top_k, N), 3.0, dtype=torch.float16, device=DEV)
+        flashnn_amd.fused_moe_a8w8_forward(a, b, c, ar, ac, w, ids.to(DEV), s.to(DEV), e.to(DEV), used.to(DEV), True, top_k,
+                                           block)
+        return c, _lib.last_kernel()
+
+    want, kernel = run(*workloads.moe_align_block_size(ids, 256, E), 256)
+    assert kernel == "gemm_a8w8_ring_kernel(moe)<256,256,4>"
+    s, e, used = workloads.moe_align_block_size(ids, BM, E)
+    got, kernel = run(s, e, used, BM)
+    assert kernel.startswith("gemm_a8w8_ring_kernel(moe") and f"<{tile_rows}," in kernel
+    assert torch.equal(got, want)
+    order = torch.randperm(int(used[0]) // BM, generator=g)
+    s2, e2 = s.clone(), e.clone()
+    s2[:int(used[0])] = s[:int(used[0])].reshape(-1, BM)[order].flatten()
+    e2[:order.numel()] = e[order]
+    assert torch.equal(run(s2, e2, used, BM)[0], want)
+    cut = (int(used[0]) // BM // 2) * BM
+    got, _ = run(s, e, torch.tensor([cut], dtype=torch.int32), BM)
+    listed = torch.zeros(M * top_k + 1, dtype=torch.bool)
+    listed[s[:cut].long()] = True
+    listed = listed[:-1].to(DEV)
+    got, want = got.reshape(M * top_k, N), want.reshape(M * top_k, N)
+    assert torch.equal(got[listed], want[listed]) and bool((got[~listed] == 3.0).all())
+
+
 @pytest.mark.parametrize("shape", [(16, 8, 1024, 1024, 2, 16), (1024, 8, 1024, 1024, 2, 64), (9, 4, 48, 80, 2, 16)])
 def test_fused_moe_a8w8_strided_operands(shape):
     """Tokens, expert weights and output that are column slices of wider buffers (the launcher passes their row and
