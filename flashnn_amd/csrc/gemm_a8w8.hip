@@ -200,9 +200,10 @@ __device__ __forceinline__ void ring_tile(const A8W8Args& p, const MoeArgs& moe,
     // from the same few memory channels: tile column c then starts p.rot * c slabs into K and goes round (the last slab,
     // which may be partial, stays the last).  Integer sums do not depend on the order.
     const int whole = (Kl + BK - 1) / BK - 1;
-    const int rot = MOE ? (n0 / BN * p.rot) % whole : 0;
+    constexpr bool ROT = MOE || BN == 128;
+    const int rot = ROT ? (n0 / BN * p.rot) % whole : 0;
     auto slab_base = [&](const int8_t* m, int kt) -> const char* {
-        if (MOE && kt < whole) kt = kt + rot - (kt + rot >= whole ? whole : 0);
+        if (ROT && kt < whole) kt = kt + rot - (kt + rot >= whole ? whole : 0);
         const uint64_t v = (uint64_t)m + (uint64_t)((int64_t)kt * BK);
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
@@ -916,6 +917,15 @@ static A8W8Args rows_from(const A8W8Args& p, int64_t m0, int m, int mode) {
 // 732 / 741; K = 7392 .. 8896: within 1 %), so they are taken up to K = 8192.
 static int group_columns(int bn, int k) { return bn >= 192 && k <= 8192 ? 8 : 4; }
 
+// Slabs by which neighbouring tile columns start apart (the kernel's rot).  Up to two rows of tiles the weights stream from
+// HBM, each piece for one tile or two, and where their rows lie a multiple of 4 KiB apart all tiles at one slab pull on the
+// same memory channels (same box, 0 / 1 slab, us: N=28672 K=8192 M=64 49.5 / 42.9, M=128 58.1 / 49.3, M=256 74.6 / 67.0;
+// N=14784 K=8192 M=100 37.5 / 32.5, M=256 49.0 / 44.2; N=22016 K=4096 M=65 26.3 / 23.7, M=256 37.5 / 35.2; steps of 3 or 11
+// slabs within 2 % of one).  More rows share the pieces through the L2 and gain nothing (M=512: within 1 %; M=2048
+// N=12288 K=4096 86.1 / 87.0), nor do rows with another stride (K = 3584, 5120, 7392, 8896, 17792: within 1 %, 7392 split
+// over two workgroups 33.9 / 34.9).
+static int rotation(const A8W8Args& p) { return p.M <= 256 && p.ldb % 4096 == 0 ? 1 : 0; }
+
 template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2>
 static void launch_mfma(A8W8Args& p, hipStream_t st) {
     p.tiles_m = (p.M + BM - 1) / BM;
@@ -923,6 +933,7 @@ static void launch_mfma(A8W8Args& p, hipStream_t st) {
     const int tiles = p.tiles_m * p.tiles_n;
     p.tiles_per_xcd = (tiles + 7) / 8;
     p.gn = group_columns(BN, p.K);
+    p.rot = rotation(p);
     note_kernel("gemm_a8w8_ring_kernel", BM, BN, WGM * 2);
     gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, WGM><<<dim3(p.tiles_per_xcd * 8), dim3(WGM * 128), 0, st>>>(p, MoeArgs{});
 }
@@ -935,6 +946,7 @@ static void launch_mfma_split(A8W8Args& p, hipStream_t st) {
     const int units = p.tiles_m * p.tiles_n * p.kparts;
     p.tiles_per_xcd = (units + 7) / 8;
     p.gn = group_columns(BN, p.K);
+    p.rot = rotation(p);
     note_kernel("gemm_a8w8_ring_kernel(split K)", BM, BN, p.kparts);
     gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, 2, true><<<dim3(p.tiles_per_xcd * 8), dim3(256), 0, st>>>(p, MoeArgs{});
 }
@@ -1052,7 +1064,9 @@ static void dispatch_band(A8W8Args& p, hipStream_t st, bool aligned, int force_b
     // 28.8 / 24.6, N=28672 30.0 / 29.8 on one box and 30.4 / 25.4 on another; N=24576 K=8192 55.3 / 45.1;
     // N=17792 K=13312 86.0 / 60.0; M=33 alike; M=24: N=24576 K=4096 30.4 / 25.3, N=17792 K=13312 60.9 / 55.9,
     // elsewhere within a few percent, the tiled kernel never behind)
-    const bool between_rounds = fast && p.M > 16 && p.M <= 64 && p.N > 16384 && p.N < 32768;
+    // (from 9 rows on where the tiled kernel starts its columns apart, see rotation: M=16 N=28672 K=8192 47.0 / 41.8,
+    // N=22016 K=4096 22.8 / 21.1; M=4: 42.9 / 41.4, 20.9 / 20.9)
+    const bool between_rounds = fast && p.M > (rotation(p) ? 8 : 16) && p.M <= 64 && p.N > 16384 && p.N < 32768;
     if (force_bm == 0 && !between_rounds && (p.M <= 64 || narrow) && launch_a8w8_skinny(p, MODE, st)) return;
     if (fast && ws.ptr) {
         if (ws.force_kparts > 1) {          // (the entry point has checked tile, parts and workspace size)

@@ -218,6 +218,24 @@ def test_a8w8_between_one_and_two_rounds_of_few_row_workgroups(M, N, K, kernel):
     assert np.array_equal(acc, O.gemm_a8w8_acc(a.numpy(), b.numpy()))
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(9, 16640, 4096, "64,128"), (65, 4112, 4096, "64,128"), (256, 12304, 4096, "128,128"),
+                                        (250, 22016, 4096, "256,128"), (100, 2048, 8192, None), (257, 4096, 4096, None)])
+def test_a8w8_tile_columns_that_start_apart(M, N, K, tile):
+    """Weight rows a multiple of 4 KiB apart, up to 256 rows: tile columns start at different slabs of K and go round, split
+    over several workgroups or not; with padded weight rows (another stride) they start together.  The same accumulators."""
+    a, b = _rand_i8((M, K), 66).to(DEV), _rand_i8((N, K + 64), 67).to(DEV)
+    plain = b[:, :K].contiguous()
+    ar, ac = torch.rand(M, device=DEV), torch.rand(N, device=DEV)
+    apart = flashnn_amd.GemmA8W8(torch.bfloat16)(a, plain, ar, ac)
+    if tile:
+        assert _lib.last_kernel() == f"gemm_a8w8_ring_kernel<{tile},4>", _lib.last_kernel()
+    out = torch.empty_like(apart)
+    launchers.hip_gemm_a8w8_forward(out, a, b[:, :K], ar, ac)
+    assert torch.equal(out, apart)
+    want = O.gemm_a8w8_acc(a[:8].cpu().numpy(), plain.cpu().numpy())
+    assert np.array_equal(launchers.hip_gemm_a8w8_int32(a, plain)[:8].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [(2, 4096, 4096, "skinny"), (16, 4096, 1024, "skinny"), (9, 1024, 11008, "skinny"),
                                           (16, 8192, 3072, "skinny"), (8, 8192, 8192, "skinny"), (3, 16384, 8192, "skinny"),
                                           (17, 4096, 4096, "panel"), (16, 4112, 4096, "panel"), (16, 8192, 3200, "panel"),
