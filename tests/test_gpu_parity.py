@@ -893,6 +893,66 @@ def test_fused_moe_a16w4_many_rows_close(shape, group, zp_kind, act_ty):
             assert (want == 3.0).all(axis=1).any() and np.array_equal((got == 3.0).all(axis=1), (want == 3.0).all(axis=1))
 
 
+@pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("group,with_zp", [(0, True), (0, False), (128, True), (128, False)])
+@pytest.mark.parametrize("shape", [
+    # M, E, output channels, K, top_k, block, tile
+    (300, 8, 2816, 512, 2, 16, "64,128"), (90, 5, 4224, 768, 3, 32, "64,128"), (1, 64, 2048, 1024, 6, 16, "64,128"),
+    (400, 4, 16384, 4096, 1, 64, "128,256"), (1300, 5, 5376, 512, 2, 64, "128,256"), (900, 2, 19200, 1280, 1, 128, "128,256")])
+def test_fused_moe_a16w4_blocks_put_together(shape, group, with_zp, act_ty):
+    """The tiled kernel over blocks of one expert put together, against float64 products of the same integers, activations and
+    tables: fp32 sums of K products (K 2^-24 of their magnitudes at most) and one rounding to 16 bits.  The bits do not hang on
+    the order of the blocks (shuffled: runs of one block, more tiles than the grid was sized for), on strided operands or on a
+    list cut in the middle, whose other rows keep their value."""
+    M, E, N, K, top_k, BM, tile = shape
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    abuf = torch.randn(M, K + 64, device=DEV, generator=g).to(act_ty)
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    sshape = (E, N) if group == 0 else (E, N, K // group)
+    scale = torch.empty(sshape, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
+    zp = torch.empty(sshape, device=DEV).uniform_(-8, 8, generator=g).to(act_ty) if with_zp else None
+    ids = torch.stack([torch.randperm(max(E, top_k))[:top_k] % E for _ in range(M)])
+    w = torch.rand(M, top_k, device=DEV, generator=g)
+    s, e, used = workloads.moe_align_block_size(ids, BM, E)
+
+    def run(a, s, e, used, mul_w=True, pad=0):
+        c = torch.full((M, top_k, N + pad), 3.0, dtype=act_ty, device=DEV)
+        flashnn_amd.fused_moe_a16w4_forward(a, b, c[:, :, :N], scale, zp, w, ids.to(DEV), s.to(DEV), e.to(DEV), used.to(DEV),
+                                            mul_w, top_k, BM)
+        assert _lib.last_kernel() == f"gemm_wo_moe_kernel{'(group tables)' if group else ''}<4,{tile}>", _lib.last_kernel()
+        assert bool((c[:, :, N:] == 3).all())
+        return c[:, :, :N]
+
+    a = abuf[:, :K].contiguous()
+    got = run(a, s, e, used)
+    for t in range(0, M * top_k, max(1, M * top_k // 40)):
+        ex = int(ids.flatten()[t])
+        nib = torch.stack([(b[ex] << 4) >> 4, b[ex] >> 4], 1).reshape(N, K).double()
+        G = 1 if group == 0 else K // group
+        z = zp[ex].double().reshape(N, G, 1) if with_zp else 0.0
+        terms = (nib.reshape(N, G, K // G) - z) * scale[ex].double().reshape(N, G, 1) * a[t // top_k].double().reshape(1, G, K // G)
+        want = terms.sum((1, 2)) * w.flatten()[t].double()
+        # the sums run over a * (c + q), c = 1032 or 136, before c and the zero point are taken off
+        off = 1048.0 if act_ty == torch.float16 else 152.0
+        mags = (a[t // top_k].double().abs().reshape(1, G, K // G).sum(2) * off * scale[ex].double().reshape(N, G)).sum(1)
+        bound = want.abs() * (2.0 ** -11 if act_ty == torch.float16 else 2.0 ** -8) * 1.01 + mags * 2.0 ** -24 * (K // G) * \
+            w.flatten()[t].double() + 1e-7
+        err = (got.reshape(M * top_k, N)[t].double() - want).abs()
+        assert bool((err <= bound).all()), (t, float((err / bound).max()))
+    assert torch.equal(run(abuf[:, :K], s, e, used, pad=9), got)
+    order = torch.randperm(int(used[0]) // BM)
+    s2, e2 = s.clone(), e.clone()
+    s2[:int(used[0])] = s[:int(used[0])].reshape(-1, BM)[order].flatten()
+    e2[:order.numel()] = e[order]
+    assert torch.equal(run(a, s2, e2, used), got)
+    cut = int(used[0]) // BM // 2 * BM
+    part = run(a, s, e, torch.tensor([cut], dtype=torch.int32)).reshape(M * top_k, N)
+    listed = torch.zeros(M * top_k + 1, dtype=torch.bool)
+    listed[s[:cut].long()] = True
+    listed = listed[:-1].to(DEV)
+    assert torch.equal(part[listed], got.reshape(M * top_k, N)[listed]) and bool((part[~listed] == 3.0).all())
+
+
 # ------------------------------------------------------------------ weight-only GEMM
 def _wo_inputs(M, N, K, group, bits, act_ty, scale_ty, with_zp, with_bias, seed):
     g = torch.Generator().manual_seed(seed)
