@@ -65,6 +65,20 @@ template <int DT> __device__ __forceinline__ float quant_in_dtype_f(float x, flo
     return rintf(bits_to_f32<DT>(f32_to_bits<DT>(t)));
 }
 
+// Two fp32 values rounded to the 16-bit type and back (bf16: one conversion instruction for the pair).  Pinned as above.
+template <int DT> __device__ __forceinline__ void round_pair(float& a, float& b) {
+    a = rounded_f32(a);
+    b = rounded_f32(b);
+    if constexpr (DT == FNN_BF16) {
+        const uint32_t pk = __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf));
+        a = __uint_as_float(pk << 16);
+        b = __uint_as_float(pk & 0xFFFF0000u);
+    } else {
+        a = f16_bits_to_f32(f32_to_f16_bits(a));
+        b = f16_bits_to_f32(f32_to_f16_bits(b));
+    }
+}
+
 // Reciprocal to hand to div_by: 1/s, or 0 for an all-zero row, whose quotients then come out as 0
 // instead of 0 * inf (so the per-element test for s == 0 can go).
 __device__ __forceinline__ float quant_rcp(float s) { return s == 0.f ? 0.f : 1.0f / s; }
@@ -77,6 +91,15 @@ __device__ __forceinline__ float quant_rcp(float s) { return s == 0.f ? 0.f : 1.
 // unclamped cast wraps to -128).
 __device__ __forceinline__ uint32_t put_biased_byte(float r, int j, uint32_t w) {
     return __builtin_amdgcn_cvt_pk_u8_f32(r + 128.f, (uint32_t)j, w);
+}
+
+// Two quotients x / s, rounded to the 16-bit type, as biased bytes j and j + 1 of w.  v_cvt_pk_u8_f32 rounds to nearest even, so
+// it is the rint as well: t + 128 is exact for a 16-bit t of at least 2^-6, and a smaller one is nowhere near a tie.
+template <int DT> __device__ __forceinline__ uint32_t put_quant_pair(float x0, float x1, float s, float r, int j, uint32_t w) {
+    float t0 = div_by(x0, s, r), t1 = div_by(x1, s, r);
+    round_pair<DT>(t0, t1);
+    w = __builtin_amdgcn_cvt_pk_u8_f32(t0 + 128.f, (uint32_t)j, w);
+    return __builtin_amdgcn_cvt_pk_u8_f32(t1 + 128.f, (uint32_t)(j + 1), w);
 }
 
 __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {

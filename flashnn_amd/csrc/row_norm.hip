@@ -145,9 +145,120 @@ __global__ __launch_bounds__(kRowThreads) void norm_vec_kernel(const NormArgs p)
             if (idx < nvec) {
                 uint32_t w[2] = {0, 0};
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    w[j >> 2] = put_biased_byte(quant_in_dtype_f<DT>(n[i][j], s, rcp), j & 3, w[j >> 2]);
+                for (int j = 0; j < 8; j += 2)
+                    w[j >> 2] = put_quant_pair<DT>(n[i][j], n[i][j + 1], s, rcp, j & 3, w[j >> 2]);
                 qr[idx] = v2u{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
+            }
+        }
+    }
+}
+
+// A workgroup walks several rows.  The next row is requested before this one is worked on, and gamma and beta (16-bit) stay in
+// registers as they came, so a row costs its own loads only and they are on their way during the arithmetic of the row
+// before.  That arithmetic is what bounds it with quantisation (about 20 vector instructions a value: four for the fp64
+// moments, nine to normalise, six to quantise; 4001 x 8192 in 29.8 us against 16 us of memory time at 6 TB/s), so values are
+// rounded in pairs.
+template <int DT, int NV, int OP, int GB>
+__global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const NormArgs p, const int rows) {
+    __shared__ double redd[2][8];       // (by turns: a slow wave may still read what the row before left)
+    __shared__ float red[2][4];
+    const int nvec = p.K >> 3;
+    v4u gv[NV], bv[OP == OP_RMS ? 1 : NV], xv[NV];
+    auto request = [&](int row) {
+        const v4u* const xr = (const v4u*)(p.x + (int64_t)row * p.ldx);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int idx = threadIdx.x + i * kRowThreads;
+            xv[i] = idx < nvec ? xr[idx] : v4u{0, 0, 0, 0};
+        }
+    };
+    request(blockIdx.x);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int idx = threadIdx.x + i * kRowThreads;
+        gv[i] = idx < nvec ? ((const v4u*)p.gamma)[idx] : v4u{0, 0, 0, 0};
+        if constexpr (OP != OP_RMS) bv[i] = idx < nvec ? ((const v4u*)p.beta)[idx] : v4u{0, 0, 0, 0};
+    }
+    int turn = 0;
+    for (int row = blockIdx.x; row < rows; row += gridDim.x, turn ^= 1) {
+        float n[NV][8];
+        double acc = 0.0, acc1 = 0.0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                n[i][2 * j] = bits_to_f32<DT>(xv[i][j] & 0xFFFFu);
+                n[i][2 * j + 1] = bits_to_f32<DT>(xv[i][j] >> 16);
+            }
+        if (row + (int)gridDim.x < rows) request(row + gridDim.x);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const double xd = (double)n[i][j];
+                acc = __builtin_fma(xd, xd, acc);
+                if constexpr (OP != OP_RMS) acc1 += xd;
+            }
+        float mul, mean = 0.f;
+        if constexpr (OP == OP_RMS) {
+            const float sum = (float)block_sum(acc, redd[turn]);
+            mul = 1.0f / sqrtf(sum / (float)p.K + p.eps);
+        } else {
+            block_sum2(acc, acc1, redd[turn]);
+            const double m64 = acc1 / (double)p.K;
+            mean = (float)m64;
+            const float var = (float)fmax(acc / (double)p.K - m64 * m64, 0.0);
+            mul = 1.0f / sqrtf(var + p.eps);
+        }
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int idx = threadIdx.x + i * kRowThreads;
+            if (idx < nvec) {
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    float y[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float g = bits_to_f32<GB>((gv[i][j >> 1] >> (16 * h)) & 0xFFFFu);
+                        if constexpr (OP == OP_RMS) {
+                            y[h] = round_dt<DT>(n[i][j + h] * mul) * g;
+                        } else {
+                            const float b = bits_to_f32<GB>((bv[i][j >> 1] >> (16 * h)) & 0xFFFFu);
+                            y[h] = ((n[i][j + h] - mean) * mul) * g + b;
+                        }
+                    }
+                    round_pair<DT>(y[0], y[1]);
+                    n[i][j] = y[0];
+                    n[i][j + 1] = y[1];
+                    if constexpr (OP == OP_LNQ) mx = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), mx);
+                }
+                if constexpr (OP != OP_LNQ) {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        o[j] = f32_to_bits<DT>(n[i][2 * j]) | (f32_to_bits<DT>(n[i][2 * j + 1]) << 16);
+                    ((v4u*)((uint16_t*)p.out + row * p.ldo))[idx] = v4u{o[0], o[1], o[2], o[3]};
+                }
+            }
+        }
+        if constexpr (OP == OP_LNQ) {
+            mx = block_max(mx, red[turn]);
+            const uint32_t sbits = f32_to_bits<DT>(mx / 127.0f);
+            const float s = bits_to_f32<DT>(sbits);
+            if (threadIdx.x == 0) p.scale[row] = (uint16_t)sbits;
+            const float rcp = quant_rcp(s);
+            v2u* qr = (v2u*)((int8_t*)p.out + row * p.ldo);
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int idx = threadIdx.x + i * kRowThreads;
+                if (idx < nvec) {
+                    uint32_t w[2] = {0, 0};
+#pragma unroll
+                    for (int j = 0; j < 8; j += 2)
+                        w[j >> 2] = put_quant_pair<DT>(n[i][j], n[i][j + 1], s, rcp, j & 3, w[j >> 2]);
+                    qr[idx] = v2u{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
+                }
             }
         }
     }
@@ -211,6 +322,26 @@ static void launch_norm(const NormArgs& p, int64_t M, hipStream_t st) {
     if (vec) {
         const int nv = (p.K / 8 + kRowThreads - 1) / kRowThreads;
         note_kernel("norm_vec_kernel", OP, nv, M <= 1024 && nv <= 4);
+        // Rows that give every lane at least 8 values and leave registers for the next row and the tables (bf16, us, one
+        // workgroup per row / at most 2048 walking them - layernorm 4001 x 8192 32.6 / 27.3, 8192 x 8192 60.9 / 50.7, 600 x 8192 10.4 /
+        // 8.4, 2100 x 2048 8.3 / 7.7; with quantisation 32.7 / 29.8, 58.7 / 52.0, 11.4 / 9.1, 9.6 / 8.6; rmsnorm 26.5 / 24.3, 50.1 /
+        // 50.2, 8.6 / 7.7, 7.2 / 6.5; 8000 x 1024, half of the lanes idle: 15.0 / 15.8, 18.7 / 19.2, 11.8 / 11.6.  Up to 8 vectors per
+        // lane take 195 registers: with quantisation 2100 x 13312 35 / 51).  1024 workgroups: 8192 x 8192 56.6 and 54.6, 2100 x 8192
+        // 18.0 / 17.8 and 19.7 / 18.5.
+        if (nv <= 4 && p.K >= 8 * kRowThreads && is16(p.gb_dtype)) {
+            const dim3 few((unsigned)(M < 2048 ? M : 2048));
+            note_kernel("norm_rows_kernel", OP, nv);
+#define FNN_NORM_ROWS(NV)                                                                                           \
+    do {                                                                                                            \
+        if (p.gb_dtype == FNN_F16) norm_rows_kernel<DT, NV, OP, FNN_F16><<<few, block, 0, st>>>(p, (int)M);         \
+        else norm_rows_kernel<DT, NV, OP, FNN_BF16><<<few, block, 0, st>>>(p, (int)M);                              \
+    } while (0)
+            if (nv <= 1) FNN_NORM_ROWS(1);
+            else if (nv <= 2) FNN_NORM_ROWS(2);
+            else FNN_NORM_ROWS(4);
+#undef FNN_NORM_ROWS
+            return;
+        }
         // up to four workgroups per CU are "few rows": every row is then resident at once either way
 #define FNN_NORM(NV)                                                                   \
     do {                                                                               \

@@ -51,10 +51,8 @@ __global__ __launch_bounds__(kRowThreads) void dynamic_quant_vec_kernel(
         if (idx < nvec) {
             uint32_t w[2] = {0, 0};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                w[j >> 1] = put_biased_byte(quant_in_dtype_f<DT>(bits_to_f32<DT>(v[i][j] & 0xFFFFu), s, rcp), 2 * (j & 1), w[j >> 1]);
-                w[j >> 1] = put_biased_byte(quant_in_dtype_f<DT>(bits_to_f32<DT>(v[i][j] >> 16), s, rcp), 2 * (j & 1) + 1, w[j >> 1]);
-            }
+            for (int j = 0; j < 4; ++j)
+                w[j >> 1] = put_quant_pair<DT>(bits_to_f32<DT>(v[i][j] & 0xFFFFu), bits_to_f32<DT>(v[i][j] >> 16), s, rcp, 2 * (j & 1), w[j >> 1]);
             qr[idx] = v2u{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
         }
     }

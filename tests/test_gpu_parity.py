@@ -893,6 +893,28 @@ def test_fused_moe_a16w4_many_rows_close(shape, group, zp_kind, act_ty):
             assert (want == 3.0).all(axis=1).any() and np.array_equal((got == 3.0).all(axis=1), (want == 3.0).all(axis=1))
 
 
+@pytest.mark.parametrize("gb_ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K", [(1, 2048), (2047, 2056), (2049, 4096), (4100, 2568), (3, 8192)])
+def test_norm_rows_walked_by_a_workgroup(M, K, ty, gb_ty):
+    """Up to three rows per workgroup, ragged and whole vectors per lane: the bits of the one-workgroup-per-row kernel, which
+    fp32 gamma and beta of the same values take, in all three operators."""
+    g = torch.Generator().manual_seed(M + K)
+    x = (torch.randn(M, K, generator=g) * 3).to(ty).to(DEV)
+    x[M // 2] = 0
+    w = torch.empty(K).uniform_(0.5, 1.5, generator=g).to(gb_ty).to(DEV)
+    b = torch.empty(K).uniform_(-0.5, 0.5, generator=g).to(gb_ty).to(DEV)
+    for op, kernel in ((lambda w, b: (launchers.hip_rmsnorm_forward(x, w, 1e-6),), 0),
+                       (lambda w, b: (launchers.hip_layer_norm_forward(x, w, b, 1e-5),), 1),
+                       (lambda w, b: launchers.hip_layer_norm_dquant_forward(x, w, b, 1e-5), 2)):
+        got = op(w, b)
+        assert _lib.last_kernel().startswith(f"norm_rows_kernel<{kernel},"), _lib.last_kernel()
+        want = op(w.float(), b.float())
+        assert _lib.last_kernel().startswith(f"norm_vec_kernel<{kernel},"), _lib.last_kernel()
+        for u, v in zip(got, want):
+            assert torch.equal(u, v)
+
+
 @pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("group,with_zp", [(0, True), (0, False), (128, True), (128, False)])
 @pytest.mark.parametrize("shape", [

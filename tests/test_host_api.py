@@ -267,3 +267,11 @@ def test_empty_calls_need_no_addresses(hip_lib):
     assert hip_lib.fnn_gemm_a8w8(null, null, null, null, null, 8, 256, 4096, 4096, 4096, 256, 0, 0, 0, null) == -1
     assert hip_lib.fnn_gemm_a16w8(null, null, null, null, null, null, 0, 256, 4096, 4096, 4096, 256, 0,
                                   0, 0, 0, 0, 0, null) == 0
+
+
+@pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
+def test_biased_byte_needs_no_rounding_of_its_own(ty):
+    """Every 16-bit quotient: 128 added in fp32 and rounded to nearest even is the rounded quotient plus 128."""
+    t = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(ty).float()
+    t = t[torch.isfinite(t) & (t.abs() <= 4096)]
+    assert torch.equal(torch.round(t + 128.0), torch.round(t) + 128.0)
