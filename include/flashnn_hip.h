@@ -377,10 +377,12 @@ int fnn_fused_moe_a8w8(void* c, const void* a, const void* b, const void* alpha_
  * N % 16 == 0, K >= 1024, block_m % 16 == 0, EM % block_m == 0 and 16-byte aligned rows; anything else
  * takes a slow guarded kernel.  The reference multiplies the dequantised weights of a K block by their scale
  * before the dot product and rounds them to the scale type; here the block's dot product is scaled
- * afterwards, in fp32.  Many routed rows per expert: with block_m a multiple of 128, 2N % 128 == 0, K % 256 == 0
- * and either group = 0 with floating zero points or group = 128 with contiguous tables of one 16-bit type
- * (zero points in the scales' type, K <= 8192) the call runs the tiled MFMA kernel over the sorted rows (128 or
- * 256 rows x 128 channels per workgroup).
+ * afterwards, in fp32.  More routed rows per expert than a pass or two of that kernel: with 2N % 128 == 0, K % 256 == 0 and
+ * either group = 0 with floating zero points or group = 128 with contiguous tables of one 16-bit type (zero points in the
+ * scales' type) the call runs tiled MFMA kernels over the sorted rows.  K <= 4096 for group = 128, block_m 16, 32, 64 or a
+ * multiple of 64: a tile is a part of one block or several consecutive blocks of one expert (128 rows x 256 channels or 64 x 128),
+ * so block_m decides the padding and not the speed.  Few tiles, or K <= 8192: block_m a multiple of 128, tiles of 128 or 256 rows
+ * x 128 channels.
  */
 int fnn_fused_moe_a16w4(void* c, const void* a, const void* b, const void* scale_b,
                         const void* zero_points, const void* topk_weights,
