@@ -59,12 +59,6 @@ template <int DT> __device__ __forceinline__ int quant_in_dtype(float x, float s
     return (int)rintf(th);
 }
 
-// The same with the result left as an integer-valued float (for the packing below).
-template <int DT> __device__ __forceinline__ float quant_in_dtype_f(float x, float s, float r) {
-    const float t = rounded_f32(div_by(x, s, r));
-    return rintf(bits_to_f32<DT>(f32_to_bits<DT>(t)));
-}
-
 // Two fp32 values rounded to the 16-bit type and back (bf16: one conversion instruction for the pair).  Pinned as above.
 template <int DT> __device__ __forceinline__ void round_pair(float& a, float& b) {
     a = rounded_f32(a);

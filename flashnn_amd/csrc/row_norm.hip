@@ -1,6 +1,6 @@
 // RMSNorm, LayerNorm and LayerNorm + per-token int8 quantisation for gfx950: the producers one step
-// before the quantised GEMMs.  One 256-thread workgroup per row; the row is read once with 16-byte
-// loads and stays in registers over the reductions.
+// before the quantised GEMMs.  A 256-thread workgroup takes a row (or several, one after the other); the
+// row is read once with 16-byte loads and stays in registers over the reductions.
 //
 //   rmsnorm            n = x * (1 / sqrt(mean(x^2) + eps)) in fp32, rounded to the input type, times
 //                      gamma, rounded to the input type (flashnn/norm.py:25-33)
