@@ -21,7 +21,7 @@
 // accumulators move between the register files).
 // 8 experts of N=28672 K=4096, groups of 128, bf16, 1024 tokens in blocks of 64: 1266 us on the panel kernel -> 775 (620
 // TFLOP/s); 2048 tokens in blocks of 128 1706 (the fold on 128 x 128 tiles) -> 1415; 64 experts N=2816 K=2048, 64 rows per
-// expert 922 -> 135; per-channel tables, N=4096 K=14336, 256 rows per expert 1264 -> 370.
+// expert 922 -> 135; per-channel tables, N=4096 K=14336, 250 rows per expert in blocks of 64 1171 -> 370.
 #include <type_traits>
 
 #include "wo_common.h"
@@ -143,18 +143,28 @@ __device__ __forceinline__ void moe_tile(const WoArgs& p, const MoeArgs& q, cons
 #pragma unroll
         for (int s = 0; s < 2; ++s) a_rd[h][s] = (wm * WTM + row16) * 256 + (((8 * h + 2 * g + s) ^ row16) << 4);
 
-    v4f outv[NA][FB], asum[FB];
+    v4f outv[NA][FB];
 #pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        asum[b] = v4f{0, 0, 0, 0};
+    for (int b = 0; b < FB; ++b)
 #pragma unroll
         for (int a = 0; a < NA; ++a) outv[a][b] = v4f{0, 0, 0, 0};
+    float czp[NA];       // per-channel tables: c + zp of the lane's channels
+    if constexpr (!GROUPS) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            const int n = n0 + wn * WTN + (a >> 1) * 32 + 2 * row16 + (a & 1);
+            czp[a] = c_off + (has_zp ? load_as_f32(p.zp, (int64_t)expert * q.stride_zp_be + n, p.zp_dtype) : 0.f);
+        }
     }
     const v4u ones = v4u{MT::one2, MT::one2, MT::one2, MT::one2};
     const v4f zero4 = v4f{0, 0, 0, 0};
 
     // One slab: all of its weights are converted first, then one activation fragment at a time is read (a fragment ahead),
-    // multiplied, and its sums folded while the MFMAs of the next fragment run.
+    // multiplied, and its sums folded while the MFMAs of the next fragment run.  Per-channel tables: the sums go on over K
+    // and the fold only takes the slab's (c + zp) * sum a off them.  Left to the end of K, the offset (1032 times the row sum in
+    // fp16) makes the fp32 sums that much longer than the result: relative error beside the output's rounding, fp16,
+    // K = 14336, activations of mean 0 / all positive: 1.1e-4 / 2.0e-4 with one fold at the end, 1.3e-5 / 2e-6 with one per
+    // slab (panel kernel 4.5e-5 / 2.1e-5; K = 1024: 1.4e-5 / 5e-6, level with it).  It costs 4 to 6 %.
     auto slab = [&](const char* sa, const char* sw, const char* tab) {
         v4u A[4][NA];
 #pragma unroll
@@ -185,7 +195,7 @@ __device__ __forceinline__ void moe_tile(const WoArgs& p, const MoeArgs& q, cons
         }
         v4f acc[2][NA], as[2];
 #pragma unroll
-        for (int b = 0; b < FB + (GROUPS ? 1 : 0); ++b) {
+        for (int b = 0; b <= FB; ++b) {
             if (b + 1 < FB) read_b(b + 1);
             if (b < FB) {
 #pragma unroll
@@ -194,29 +204,29 @@ __device__ __forceinline__ void moe_tile(const WoArgs& p, const MoeArgs& q, cons
                     if constexpr (GROUPS) {
 #pragma unroll
                         for (int a = 0; a < NA; ++a) acc[b & 1][a] = MT::mma(bv, A[ks][a], ks == 0 ? zero4 : acc[b & 1][a]);
-                        as[b & 1] = MT::mma(bv, ones, ks == 0 ? zero4 : as[b & 1]);
                     } else {
 #pragma unroll
                         for (int a = 0; a < NA; ++a) outv[a][b] = MT::mma(bv, A[ks][a], outv[a][b]);
-                        asum[b] = MT::mma(bv, ones, asum[b]);
                     }
+                    as[b & 1] = MT::mma(bv, ones, ks == 0 ? zero4 : as[b & 1]);
                 }
             }
-            if constexpr (GROUPS) {
-                if (b > 0) {
+            if (b > 0) {
 #pragma unroll
-                    for (int a = 0; a < NA; ++a)
+                for (int a = 0; a < NA; ++a)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            outv[a][b - 1][r] += sc[a] * (acc[(b - 1) & 1][a][r] - zc[a] * as[(b - 1) & 1][r]);
-                }
-                if (b < FB) {
-                    if (b + 1 < FB) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-                    for (int i = 0; i < 4 * (NA + 1); ++i) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                    for (int r = 0; r < 4; ++r) {
+                        const float sum = as[(b - 1) & 1][r];
+                        if constexpr (GROUPS) outv[a][b - 1][r] += sc[a] * (acc[(b - 1) & 1][a][r] - zc[a] * sum);
+                        else outv[a][b - 1][r] = __builtin_fmaf(-czp[a], sum, outv[a][b - 1][r]);
                     }
+            }
+            if (b < FB) {
+                if (b + 1 < FB) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+                for (int i = 0; i < 4 * (NA + 1); ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, GROUPS ? 2 : 1, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -263,11 +273,10 @@ __device__ __forceinline__ void moe_tile(const WoArgs& p, const MoeArgs& q, cons
         for (int a = 0; a < NA; ++a) {
             const int n = n0 + wn * WTN + (a >> 1) * 32 + 2 * row16 + (a & 1);
             const float sc = load_as_f32(p.scale, (int64_t)expert * q.stride_scale_be + n, p.scale_dtype);
-            const float zc = c_off + (has_zp ? load_as_f32(p.zp, (int64_t)expert * q.stride_zp_be + n, p.zp_dtype) : 0.f);
 #pragma unroll
             for (int b = 0; b < FB; ++b)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) outv[a][b][r] = sc * (outv[a][b][r] - zc * asum[b][r]);
+                for (int r = 0; r < 4; ++r) outv[a][b][r] *= sc;
         }
     }
 

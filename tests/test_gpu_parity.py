@@ -915,6 +915,16 @@ def test_norm_rows_walked_by_a_workgroup(M, K, ty, gb_ty):
             assert torch.equal(u, v)
 
 
+def _moe_a16w4_exact(a, packed, scale, zp):
+    """One routed row in 64 bits: a [K], packed [N/2, K] nibble pairs, scale and zp (or None) [N] or [N, K / group]."""
+    K = a.shape[0]
+    N, G = scale.shape[0], 1 if scale.dim() == 1 else scale.shape[1]
+    nib = torch.stack([(packed << 4) >> 4, packed >> 4], 1).reshape(N, G, K // G).double()
+    if zp is not None:
+        nib = nib - zp.double().reshape(N, G, 1)
+    return ((nib * scale.double().reshape(N, G, 1)).reshape(N, K) * a.double()).sum(1)
+
+
 @pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("group,with_zp", [(0, True), (0, False), (128, True), (128, False)])
 @pytest.mark.parametrize("shape", [
@@ -973,6 +983,36 @@ def test_fused_moe_a16w4_blocks_put_together(shape, group, with_zp, act_ty):
     listed[s[:cut].long()] = True
     listed = listed[:-1].to(DEV)
     assert torch.equal(part[listed], got.reshape(M * top_k, N)[listed]) and bool((part[~listed] == 3.0).all())
+
+
+@pytest.mark.parametrize("K,block", [(14336, 16), (14336, 64), (14336, 256), (1024, 16)])
+def test_fused_moe_a16w4_per_channel_error_does_not_grow_with_k(K, block):
+    """Per-channel tables and activations that do not cancel (all positive, as behind a ReLU): what the tiled kernel adds to
+    the rounding of the output (fp16: bf16's hides it).  The nibbles ride on an offset c, so a slab of 128 carries sums of 128
+    c mean|a|; each of its roundings (taken as eight: four MFMAs, the fold, and what an MFMA rounds inside; twice the whole is
+    allowed) is at most 2^-24 of them, and the slabs' errors add up as independent ones do."""
+    T, E, N, top_k, act_ty = 200, 4, 4096, 2, torch.float16
+    g = torch.Generator(device=DEV).manual_seed(K + block)
+    a = torch.randn(T, K, device=DEV, generator=g).abs().to(act_ty)
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    scale = torch.empty(E, N, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
+    zp = torch.randint(-8, 8, (E, N), device=DEV, generator=g).to(act_ty)
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), top_k, dim=-1)[1].to(torch.int32)
+    w = torch.ones(T, top_k, device=DEV)
+    s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+    c = torch.empty(T, top_k, N, dtype=act_ty, device=DEV)
+    flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, False, top_k, block)
+    assert _lib.last_kernel().startswith("gemm_wo_moe_kernel<4,"), _lib.last_kernel()
+    rows = range(0, T * top_k, 25)
+    want = torch.stack([_moe_a16w4_exact(a[t // top_k], b[ex], scale[ex], zp[ex])
+                        for t in rows for ex in [int(ids.flatten()[t])]])
+    norm = float(want.norm())
+    err = float((c.reshape(T * top_k, N)[list(rows)].double() - want).norm()) / norm
+    rounding = float((want.to(act_ty).double() - want).norm()) / norm
+    slab = 128 * 1048.0 * float(a.double().mean())
+    added = 2 * 2.0 ** -24 * slab * (8 * K / 128) ** 0.5 * float(scale.double().square().mean().sqrt()) / float(
+        want.square().mean().sqrt())
+    assert err ** 2 <= rounding ** 2 * (1 + 1e-3) + added ** 2, (err, rounding, added)
 
 
 # ------------------------------------------------------------------ weight-only GEMM
