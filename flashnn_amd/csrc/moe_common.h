@@ -86,14 +86,14 @@ struct MoeTiles {
     }
 };
 
-// What the host can say about the routing without reading it: the sorted list holds every routed row and up to
-// block_m - 1 padding rows per expert, which gives the number of experts it was made for.  An estimate (a caller may cut
-// its list): used for grid sizes and prices only.
+// What the host can say about the routing without reading it.  A sorted list as callers allocate it holds every routed row
+// and block_m - 1 padding rows per expert, rounded up to whole blocks, which gives the number of experts.  A list cut to the
+// rows in use has less padding: with less than one expert's worth it says nothing, and every block is then taken for an expert
+// of its own, so that tiles stay within what the caller sorted for.  An estimate: used for grid sizes and prices only.
 inline int64_t moe_experts_estimate(const MoeArgs& q) {
     const int64_t blocks = q.EM / q.block_m, pad = (int64_t)q.EM - q.num_valid;
-    if (pad <= 0 || q.block_m < 2) return 1;
-    const int64_t e = (pad + q.block_m - 2) / (q.block_m - 1);
-    return e < blocks ? e : (blocks > 0 ? blocks : 1);
+    const int64_t e = q.block_m > 1 ? pad / (q.block_m - 1) : 0;
+    return e >= 1 && e < blocks ? e : (blocks > 0 ? blocks : 1);
 }
 // ... and so the number of tiles of bm rows
 inline int64_t moe_tiles_estimate(const MoeArgs& q, int bm) {

@@ -1015,6 +1015,37 @@ def test_fused_moe_a16w4_per_channel_error_does_not_grow_with_k(K, block):
     assert err ** 2 <= rounding ** 2 * (1 + 1e-3) + added ** 2, (err, rounding, added)
 
 
+@pytest.mark.parametrize("kind,E,R,N,K,block,kernel", [
+    ("a8w8", 64, 32, 2816, 1024, 32, "gemm_a8w8_ring_kernel(moe, blocks together)<64,128,4>"),
+    ("a16w4", 8, 16, 20480, 1024, 16, "gemm_wo_panel_kernel(moe)<4,1,4>")])
+def test_fused_moe_lists_cut_to_the_rows_in_use(kind, E, R, N, K, block, kernel):
+    """R rows for every expert, whole blocks of them, and the sorted list without its unused tail: no padding tells how many
+    experts there are.  The same kernel and bits as with the list as it is allocated."""
+    g = torch.Generator(device=DEV).manual_seed(E + K)
+    M = E * R // 2
+    ids = (torch.arange(2 * M, device=DEV) % E).reshape(M, 2).to(torch.int32)
+    w = torch.rand(M, 2, device=DEV, generator=g)
+    s, e, used = workloads.moe_align_block_size(ids.cpu(), block, E)
+    assert int(used[0]) == 2 * M
+    if kind == "a8w8":
+        a = torch.randint(-128, 128, (M, K), dtype=torch.int8, device=DEV, generator=g)
+        b = torch.randint(-128, 128, (E, N, K), dtype=torch.int8, device=DEV, generator=g)
+        tables = (torch.rand(M, device=DEV, generator=g) * 0.05, torch.rand(E, N, device=DEV, generator=g) * 0.05)
+        op = flashnn_amd.fused_moe_a8w8_forward
+    else:
+        a = torch.randn(M, K, device=DEV, generator=g).half()
+        b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+        tables = ((torch.rand(E, N, device=DEV, generator=g) * 0.01).half(), None)
+        op = flashnn_amd.fused_moe_a16w4_forward
+    got = []
+    for n in (s.numel(), 2 * M):
+        c = torch.empty(M, 2, N, dtype=torch.float16, device=DEV)
+        op(a, b, c, *tables, w, ids, s[:n].to(DEV), e[:n // block].to(DEV), used.to(DEV), True, 2, block)
+        assert _lib.last_kernel() == kernel, (n, _lib.last_kernel())
+        got.append(c)
+    assert torch.equal(*got)
+
+
 # ------------------------------------------------------------------ weight-only GEMM
 def _wo_inputs(M, N, K, group, bits, act_ty, scale_ty, with_zp, with_bias, seed):
     g = torch.Generator().manual_seed(seed)
