@@ -71,16 +71,19 @@ struct OptionalStage<false, BYTES> {
 };
 
 // The kernel's own arguments read again from where the launch put them.  The tile code inside a loop gets them so: left to
-// the compiler every argument that the loop needs again stays in scalar registers over the tile (70 of them spilled,
-// and with them 27 vector registers of the 256x256 tile).
+// the compiler every argument that the loop needs again stays in scalar registers over the tile (57 of them spilled,
+// and with them 15 vector registers of the 256x256 tile).  Read as 8-byte words: a byte-wise copy has no alignment that
+// scalar loads could use.
 struct Kernargs { A8W8Args p; MoeArgs moe; };
 __device__ __forceinline__ Kernargs kernargs() {
-    typedef const __attribute__((address_space(4))) char* const_ptr_t;
+    typedef const __attribute__((address_space(4))) uint64_t* const_ptr_t;
     const_ptr_t k = (const_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(k));
-    Kernargs r;
-    __builtin_memcpy(&r, k, sizeof(r));
-    return r;
+    static_assert(sizeof(Kernargs) % 8 == 0 && alignof(Kernargs) == 8, "copied in words, laid out as the kernel's arguments");
+    struct Words { uint64_t w[sizeof(Kernargs) / 8]; } words;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(Kernargs) / 8); ++i) words.w[i] = k[i];
+    return __builtin_bit_cast(Kernargs, words);
 }
 
 // SPLIT: the workgroups of the grid are units, kparts per tile, each the tile's product over its own range
@@ -100,7 +103,7 @@ __device__ __forceinline__ Kernargs kernargs() {
 // a few blocks of one expert (MoeTiles); padding rows read activation row 0 and store nothing.
 //
 // One tile: rows m0 .. of the tile (MOE: sorted rows, those from row_end on are padding), columns n0 ..; part kpart of K.
-template <int BM, int BN, int MODE, bool PAIR, int WGM, bool SPLIT, bool MOE>
+template <int BM, int BN, int MODE, bool PAIR, int WGM, bool SPLIT, bool MOE, bool LOOP>
 __device__ __forceinline__ void ring_tile(const A8W8Args& p, const MoeArgs& moe, const int t, const int kpart, const int m0,
                                           const int n0, const int row_end, const int expert, const int tid) {
     static_assert(!MOE || (!SPLIT && MODE != OUT_I32), "the gathered form has no split and no raw output");
@@ -574,7 +577,7 @@ __device__ __forceinline__ void ring_tile(const A8W8Args& p, const MoeArgs& moe,
         // the three instructions of a fragment row the wave's whole 192-byte (WTN * 2) piece of them.  No
         // LDS transposition, no barrier between the waves.
         static_assert(FN % 2 == 0, "weight fragments are stored in pairs");
-        const Kernargs again = MOE ? kernargs() : Kernargs{p, moe};
+        const Kernargs again = LOOP ? kernargs() : Kernargs{p, moe};
         const A8W8Args& p = again.p;
         const MoeArgs& moe = again.moe;
         asm volatile("" ::: "memory");
@@ -726,14 +729,22 @@ __device__ __forceinline__ void ring_tile(const A8W8Args& p, const MoeArgs& moe,
     }
 }
 
-template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2, bool SPLIT = false, bool MOE = false>
+// The forms of the kernel.  MOE_WHOLE: blocks of the tile's height and more, so a tile is a part of one block, the grid holds
+// every tile that there can be, and the kernel is straight-line code.  MOE_BLOCKS: blocks put together, which takes a search
+// before the tile and, because the host can only estimate the number of tiles, a loop around it.  The two are apart because
+// the loop costs registers: 256x256 tile, 2 of them spilled without it and 9 with it, 16 where it carried both forms.
+// Blocks of 256, 8 experts N=28672 K=4096, 4096 tokens, us: 950 in the loop, 882 without (2048 tokens 553 / 500; K=14336
+// N=4096 470 / 445).
+enum MoeForm { MOE_NONE, MOE_WHOLE, MOE_BLOCKS };
+
+template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2, bool SPLIT = false, MoeForm FORM = MOE_NONE>
 __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Args p, const MoeArgs moe) {
     const int xcd = blockIdx.x & 7;
     // tiles are numbered in groups of gn tile columns, the column fastest within a group: the 32 workgroups
     // an XCD runs at a time then cover 32 / gn tile rows x gn tile columns whatever M is, and fetch
     // (32 / gn) * BM + gn * BN operand rows per slab into its L2 instead of tiles_m*BM + BN.  gn = 8 for the tiles
     // of 192 and 256 columns, 4 for the narrower ones (measured, see the launchers).
-    auto place = [&](int t, int tiles_m, int& tile_m, int& tile_n) {
+    auto place = [](const A8W8Args& p, int t, int tiles_m, int& tile_m, int& tile_n) __attribute__((always_inline)) {
         const int grp = t / (p.gn * tiles_m);
         const int rem = t - grp * (p.gn * tiles_m);
         const int gw = min(p.gn, p.tiles_n - grp * p.gn);
@@ -741,34 +752,45 @@ __global__ __launch_bounds__(WGM * 128) void gemm_a8w8_ring_kernel(const A8W8Arg
         tile_m = rem / gw;
     };
     int tile_m, tile_n;
-    if constexpr (MOE) {
+    if constexpr (FORM == MOE_BLOCKS) {
         // The number of tiles is known on the device only.  The grid is the host's estimate of it (p.tiles_per_xcd
         // workgroups per XCD); where there are more, workgroups take a second tile.
         int slot = blockIdx.x >> 3;
         for (;;) {
-            const MoeTiles<BM> map(moe);
-            const int tiles = map.tiles * p.tiles_n, per_xcd = (tiles + 7) / 8;
-            const int t = xcd * per_xcd + slot;
-            if (slot >= per_xcd || t >= tiles) return;
-            place(t, map.tiles, tile_m, tile_n);
-            int m0, rows, expert;
-            map.find(tile_m, m0, rows, expert);
             const Kernargs k = kernargs();
             int tid = threadIdx.x;
             asm volatile("" : "+v"(tid));          // (so that what a lane derives from its number is not kept either)
-            ring_tile<BM, BN, MODE, PAIR, WGM, SPLIT, MOE>(k.p, k.moe, t, 0, m0, tile_n * BN, m0 + rows, expert, tid);
-            slot += p.tiles_per_xcd;
+            const MoeTiles<BM> map(k.moe, tid & 63);
+            const int tiles = map.tiles * k.p.tiles_n, per_xcd = (tiles + 7) / 8;
+            const int t = xcd * per_xcd + slot;
+            if (slot >= per_xcd || t >= tiles) return;
+            place(k.p, t, map.tiles, tile_m, tile_n);
+            int m0, rows, expert;
+            map.find(tile_m, m0, rows, expert);
+            slot += k.p.tiles_per_xcd;
+            const bool more = slot < per_xcd;
+            ring_tile<BM, BN, MODE, PAIR, WGM, false, true, true>(k.p, k.moe, t, 0, m0, tile_n * BN, m0 + rows, expert, tid);
+            if (!more) return;                      // (the usual case: nobody waits for the stores)
             __builtin_amdgcn_s_waitcnt(0x0070);     // this tile's stores are out, and nobody reads its LDS any more
             __syncthreads();
         }
+    } else if constexpr (FORM == MOE_WHOLE) {
+        const MoeTiles<BM, true> map(moe, threadIdx.x & 63);
+        const int slot = blockIdx.x >> 3, tiles = map.tiles * p.tiles_n, per_xcd = (tiles + 7) / 8;
+        const int t = xcd * per_xcd + slot;
+        if (slot >= per_xcd || t >= tiles) return;
+        place(p, t, map.tiles, tile_m, tile_n);
+        int m0, rows, expert;
+        map.find(tile_m, m0, rows, expert);
+        ring_tile<BM, BN, MODE, PAIR, WGM, false, true, false>(p, moe, t, 0, m0, tile_n * BN, m0 + rows, expert, threadIdx.x);
     } else {
         const int unit = xcd * p.tiles_per_xcd + (blockIdx.x >> 3);   // (tiles_per_xcd counts units where SPLIT)
         if ((blockIdx.x >> 3) >= p.tiles_per_xcd || unit >= p.tiles_m * p.tiles_n * (SPLIT ? p.kparts : 1)) return;
         // the units of a tile are neighbours in this numbering: they run on one XCD, at about the same time
         const int t = SPLIT ? unit / p.kparts : unit;
-        place(t, p.tiles_m, tile_m, tile_n);
-        ring_tile<BM, BN, MODE, PAIR, WGM, SPLIT, MOE>(p, moe, t, SPLIT ? unit - t * p.kparts : 0, tile_m * BM, tile_n * BN,
-                                                       p.M, 0, threadIdx.x);
+        place(p, t, p.tiles_m, tile_m, tile_n);
+        ring_tile<BM, BN, MODE, PAIR, WGM, SPLIT, false, false>(p, moe, t, SPLIT ? unit - t * p.kparts : 0, tile_m * BM,
+                                                                tile_n * BN, p.M, 0, threadIdx.x);
     }
 }
 
@@ -1153,12 +1175,26 @@ static void launch_mfma_moe(A8W8Args& p, const MoeArgs& q, hipStream_t st) {
     // 305.  N = 8192 K = 8192: 113 / 102 / 103; 136 / 109 / 118; 210 / 202 / 209; 501 / 497 / 522.  With more than one tile
     // row per expert the wide step takes tiles that share activation rows too far apart.  K = 7168, 14336: no difference)
     p.rot = p.ldb % 4096 != 0 ? 0 : BM == 64 ? 11 : 1;
-    note_kernel(q.block_m < BM ? "gemm_a8w8_ring_kernel(moe, blocks together)" : "gemm_a8w8_ring_kernel(moe)", BM, BN, 4);
-    gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, 2, false, true><<<dim3(p.tiles_per_xcd * 8), dim3(256), 0, st>>>(p, q);
+    const dim3 grid(p.tiles_per_xcd * 8), block(256);
+    if (q.block_m < BM) {
+        note_kernel("gemm_a8w8_ring_kernel(moe, blocks together)", BM, BN, 4);
+        gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, 2, false, MOE_BLOCKS><<<grid, block, 0, st>>>(p, q);
+    } else {
+        note_kernel("gemm_a8w8_ring_kernel(moe)", BM, BN, 4);
+        gemm_a8w8_ring_kernel<BM, BN, MODE, PAIR, 2, false, MOE_WHOLE><<<grid, block, 0, st>>>(p, q);
+    }
 }
 
 // Tile heights that the block size allows: the tile is a part of a block, or whole blocks make up the tile.
 static bool moe_tile_fits(const MoeArgs& q, int bm) { return q.block_m >= 16 && (q.block_m % bm == 0 || bm % q.block_m == 0); }
+
+// Rounds of tiles of bm x bm that a call makes with per_round of them at a time, the rows of an expert taken as spread round
+// their mean the way an even random routing spreads them.
+static double moe_rounds(const A8W8Args& p, const MoeArgs& q, int bm, int per_round) {
+    const double experts = (double)moe_experts_estimate(q), mean = (double)q.num_valid / experts, off = 1.2 * sqrt(mean);
+    const double tall = (ceil((mean - off) / bm) + ceil(mean / bm) + ceil((mean + off) / bm)) / 3.0;
+    return experts * tall * ((p.N + bm - 1) / bm) / per_round;
+}
 
 // The height of the tiles.  Blocks of a multiple of 128 rows keep tiles of at least 128, of 256 rows those of 256 (what the
 // caller sorted for).  Else by the mean number of routed rows per expert (estimated, moe_experts_estimate), where the
@@ -1168,11 +1204,23 @@ static bool moe_tile_fits(const MoeArgs& q, int bm) { return q.block_m >= 16 && 
 // 205 / 282 | 215 / 198 / 238 | 128 / 105 / 158; 100 rows 261 / 212 / 283 | 251 / 237 / 237 (128 rows) | 132 / 113 / 160 |
 // 114 / 98 / 128; 150 rows 314 / 303 / 291 | - | 169 / 150 / 164; 256 rows 429 / 366 / 361 | 375 / 327 / 322 | 232 / 221 /
 // 181 | 170 / 155 / 136 (192 rows); 1024 rows 1375 / 1128 / 999 | - | 710 / 557 / 509 | 274 / 261 / 259 (384 rows).
+// Tiles of 256 x 256 run one to a CU, in whole rounds; those of 128 x 128 two to a CU, and what is left over of a round runs
+// beside the end of the one before.  A round of the first takes 1.6 times one of the second, so a little more than a whole
+// number of rounds goes to the smaller tiles (256-row / 128-row tiles, us: 8 experts N=4096 K=7168, 512 rows per expert, 1.2
+// rounds, blocks of 128 163 / 128, of 64 162 / 133; 1024 rows, 2.2 rounds, 255 / 230; 64 experts N=2816 K=2048, 281 rows, 5.5
+// rounds, 208 / 170; 8 experts N=28672 K=4096, 1024 rows, 15.2 rounds, 913 / 994).  Long rows pay for the taller tile all
+// the same (N=4096 K=14336, 2.2 rounds 470 / 521).  Blocks of 128, which need no search with tiles of their own height, go to
+// the taller one only where its rows are well filled (8 experts N=24576 K=2048, 275 rows 205 / 179; 32 experts N=8192 K=2048, 325
+// rows 282 / 250).
 static int moe_tile_rows(const A8W8Args& p, const MoeArgs& q) {
     const int least = q.block_m % 256 == 0 ? 256 : q.block_m % 128 == 0 ? 128 : 64;
     const double mean = (double)q.num_valid / (double)moe_experts_estimate(q);
     int bm = mean <= 56 ? 64 : mean < 144 ? 128 : 256;
     while (bm > least && (!moe_tile_fits(q, bm) || moe_tiles_estimate(q, bm) * ((p.N + bm - 1) / bm) < 256)) bm /= 2;
+    if (bm == 256 && least < 256 && p.K < 8192) {
+        const double whole = ceil(moe_rounds(p, q, 256, 256) - 0.05);
+        if (whole > 1.0 && (least == 128 ? 1.66 : 1.5) * whole > moe_rounds(p, q, 128, 512) + 0.25) bm = 128;
+    }
     return bm > least ? bm : least;
 }
 

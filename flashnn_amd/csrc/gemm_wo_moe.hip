@@ -311,7 +311,7 @@ __global__ __launch_bounds__(WGM * 256, 2) void gemm_wo_moe_kernel(const WoArgs 
     // channel tile fastest within a group.  The number of tiles is known on the device only: the grid is the host's estimate
     // of it, and where there are more, workgroups take a second tile.
     const int per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7;
-    const MoeTiles<BM> map(q);
+    const MoeTiles<BM> map(q, threadIdx.x & 63);
     const int cols = p.N / BN, all = map.tiles * cols, mine = (all + 7) / 8;
     for (int slot = blockIdx.x >> 3; slot < mine; slot += per_xcd) {
         const int t = xcd * mine + slot;

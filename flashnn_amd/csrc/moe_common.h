@@ -27,20 +27,22 @@ struct MoeArgs {
 // output - does not hang on the block size that the caller sorted for.  Where an expert's blocks end, and so how many tiles
 // there are, is read from expert_ids by every wave for itself: 64 blocks per step, four steps' loads in flight (256
 // blocks: one L2 latency, about 1 us before a tile of 40 to 60 us).
-template <int BM>
+// WHOLE: the caller knows that blocks are of BM rows and more; the search is not compiled in then.
+template <int BM, bool WHOLE = false>
 struct MoeTiles {
     const MoeArgs& q;
+    const int lane;
     int blocks, tiles;       // blocks in use and tiles that they make
 
-    __device__ __forceinline__ explicit MoeTiles(const MoeArgs& args) : q(args) {
+    __device__ __forceinline__ MoeTiles(const MoeArgs& args, int lane_) : q(args), lane(lane_) {
         const int used = min(q.ntpp[0], q.EM);
         blocks = __builtin_amdgcn_readfirstlane((used + q.block_m - 1) / q.block_m);
-        tiles = q.block_m >= BM ? blocks * (q.block_m / BM) : scan(-1);
+        tiles = WHOLE || q.block_m >= BM ? blocks * (q.block_m / BM) : scan(-1);
     }
 
     // the number of tiles (want < 0), or the first block of tile `want`
     __device__ __forceinline__ int scan(int want) const {
-        const int lane = threadIdx.x & 63, r = BM / q.block_m;
+        const int r = BM / q.block_m;
         int count = 0, last_expert = 0, run = 0;        // run: first block of the expert's blocks that are being walked
         for (int base = 0; base < blocks; base += 256) {
             int e[4];
@@ -50,7 +52,8 @@ struct MoeTiles {
             for (int c = 0; c < 4; ++c) {
                 const int first = base + 64 * c, blk = first + lane;
                 if (first >= blocks) break;
-                const int before = __shfl_up(e[c], 1, 64);
+                // the lane before's value (wave_shr:1 - a shuffle keeps the lane's byte address in a register over the tile)
+                const int before = __builtin_amdgcn_update_dpp(0, e[c], 0x138, 0xF, 0xF, false);
                 const bool starts = blk < blocks && (blk == 0 || e[c] != (lane == 0 ? last_expert : before));
                 const uint64_t runs = __ballot(starts);
                 const uint64_t here = runs & (~0ull >> (63 - lane));
@@ -71,12 +74,12 @@ struct MoeTiles {
 
     // first sorted row of a tile, how many of its rows belong to it, and their expert
     __device__ __forceinline__ void find(int tile, int& m0, int& rows, int& expert) const {
-        if (q.block_m >= BM) {
+        if (WHOLE || q.block_m >= BM) {
             m0 = tile * BM;
             rows = BM;
             expert = q.expert_ids[m0 / q.block_m];
         } else {
-            const int lane = threadIdx.x & 63, r = BM / q.block_m, b = scan(tile);
+            const int r = BM / q.block_m, b = scan(tile);
             const int e = q.expert_ids[min(b + lane, blocks - 1)];
             expert = __builtin_amdgcn_readfirstlane(e);
             const uint64_t same = __ballot(lane < r && b + lane < blocks && e == expert);

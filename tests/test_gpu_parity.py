@@ -738,6 +738,32 @@ def test_fused_moe_a8w8_blocks_put_together(shape):
     assert torch.equal(got[listed], want[listed]) and bool((got[~listed] == 3.0).all())
 
 
+@pytest.mark.parametrize("M,E,N,K,block,kernel", [
+    (2048, 8, 4096, 1024, 128, "(moe)<128,128,4>"),                       # 1.2 rounds of 256-row tiles
+    (2048, 8, 4096, 1024, 64, "(moe, blocks together)<128,128,4>"),
+    (2048, 8, 4096, 8192, 128, "(moe, blocks together)<256,256,4>"),      # .. of long rows
+    (1800, 8, 4096, 1024, 128, "(moe, blocks together)<256,256,4>"),      # one round
+    (2048, 8, 4096, 1024, 256, "(moe)<256,256,4>")])
+def test_fused_moe_a8w8_tile_height_by_rounds(M, E, N, K, block, kernel):
+    """A little more than a whole number of rounds of the tallest tile goes to the smaller one; the same bits as blocks of 16."""
+    g = torch.Generator(device=DEV).manual_seed(M + K + block)
+    a = torch.randint(-128, 128, (M, K), dtype=torch.int8, device=DEV, generator=g)
+    b = torch.randint(-128, 128, (E, N, K), dtype=torch.int8, device=DEV, generator=g)
+    ar, ac = torch.rand(M, device=DEV, generator=g) * 0.05, torch.rand(E, N, device=DEV, generator=g) * 0.05
+    ids = torch.topk(torch.rand(M, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.rand(M, 2, device=DEV, generator=g)
+
+    def run(block):
+        s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+        c = torch.empty(M, 2, N, dtype=torch.bfloat16, device=DEV)
+        flashnn_amd.fused_moe_a8w8_forward(a, b, c, ar, ac, w, ids, s, e, used, True, 2, block)
+        return c, _lib.last_kernel()
+
+    got, name = run(block)
+    assert name == "gemm_a8w8_ring_kernel" + kernel
+    assert torch.equal(got, run(16)[0])
+
+
 @pytest.mark.parametrize("shape", [(16, 8, 1024, 1024, 2, 16), (1024, 8, 1024, 1024, 2, 64), (9, 4, 48, 80, 2, 16)])
 def test_fused_moe_a8w8_strided_operands(shape):
     """Tokens, expert weights and output that are column slices of wider buffers (the launcher passes their row and
