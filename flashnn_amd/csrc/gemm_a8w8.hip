@@ -1231,6 +1231,31 @@ static void launch_moe_tiled_t(A8W8Args& p, const MoeArgs& q, int bm, hipStream_
     else launch_mfma_moe<64, 128, MODE>(p, q, st);
 }
 
+// Blocks of 16 and 32 rows on which the few-row kernel, whose workgroups own 16 to 64 channels and read an expert's weights
+// once per block, is ahead of 64-row tiles (both forced under a captured graph, few-row kernel / tiles, us).
+//  * Few tiles of long rows leave most CUs without one.  N=4096, 8 experts, few-row kernel ahead by a factor of, K=14336 / 7168:
+//    blocks of 16, 1 token 1.24 / 1.09, 2 tokens 1.10 / 1.00, 3 tokens 0.96 / 0.91; blocks of 32, 1 token 1.05 / 0.93, 2 tokens 0.68 /
+//    0.62.  Blocks of 64, which the kernel reads 16 rows at a time there, never: 0.62 and less.
+//  * Wide layers and a little more than one long tile per CU, where the second on some CUs decides: 1.10 to 1.17 (16 experts
+//    N=10752 K=6144, 1 token), 1.14 to 1.20 (N=10240 K=8192, 2 tokens).
+//  * Many tiles of wide layers whose weight rows lie a multiple of 4 KiB apart, one block per expert: both stream the weights, and
+//    the narrower workgroups do it better.  us, 8 experts N=28672 K=4096, blocks of 16: 8 tokens 138 / 149, 16 tokens 145 / 151, 24
+//    tokens level, 64 tokens 0.75; blocks of 32: 16 tokens 140 / 151, 64 tokens level; 16 experts N=12288 97.6 / 107 (6
+//    tokens), 95 / 107 (8 tokens, blocks of 32); N=14336 75 / 82 (8 tokens); K=8192 N=28672 1.07 (4 tokens), N=10240 1.11
+//    (12 tokens).  Of other strides (K = 2048, 3072, 5120, 6144) and narrower layers (N=8192 K=4096 in blocks of 32: 0.9)
+//    the tiles are level or ahead, and with few experts reached (N=28672, 2 tokens: 69.5 / 65.7).
+static bool moe_few_rows_ahead(const A8W8Args& p, const MoeArgs& q) {
+    if (q.block_m > 32 || p.N % 16 != 0) return false;
+    const double experts = (double)moe_experts_estimate(q), mean = (double)q.num_valid / experts;
+    const double reached = experts * (1.0 - pow(1.0 - 1.0 / experts, (double)q.num_valid));
+    const double tiles = reached * ((p.N + 127) / 128);
+    if (tiles * (q.block_m / 16) < (p.K >= 8192 ? 150 : p.K >= 6144 ? 110 : 0)) return true;
+    if (p.N < 10240) return false;
+    if (p.K >= 6144 && tiles >= 256 && tiles < 400) return true;
+    const double least = q.block_m == 16 ? 0.75 : 0, most = q.block_m == 16 ? 6 : 16;
+    return p.ldb % 4096 == 0 && tiles >= 600 && mean >= least && mean <= most;
+}
+
 static bool launch_a8w8_moe_tiled(A8W8Args& p, const MoeArgs& q, int mode, hipStream_t st) {
     constexpr int64_t kLimit = (1LL << 31) - 1;
     const int64_t rows = (q.num_valid + q.top_k - 1) / q.top_k;          // activation rows
@@ -1240,14 +1265,7 @@ static bool launch_a8w8_moe_tiled(A8W8Args& p, const MoeArgs& q, int mode, hipSt
                     ((uintptr_t)p.b % 16) == 0 && ((uintptr_t)p.out % 16) == 0 && rows * p.lda <= kLimit &&
                     (int64_t)p.N * p.ldb <= kLimit && moe_tiles_estimate(q, 64) * ((p.N + 127) / 128) <= kLimit;
     if (!ok) return false;
-    // Few tiles of long rows leave most CUs without one: the few-row kernel, whose workgroups own 16 to 64 channels, is ahead
-    // (8 experts, N = 4096 K = 14336, blocks of 16, few-row kernel / 64-row tiles, us: 1 token 41 / 58, 2 tokens 51 / 63, 3
-    // tokens 62 / 67, 4 tokens 80 / 71, 16 tokens 99 / 87, 64 tokens 142 / 88; N = 2816 K = 2048, 64 experts, 6 per token: 1
-    // token 24 / 20, 64 tokens 159 / 79; N = 28672 K = 4096: 1 token 69 / 49, 8 tokens 150 / 160, 16 tokens 165 / 168, 64
-    // tokens 229 / 175; N = 12288 K = 4096, 16 experts: 1 token 35 / 26, 64 tokens 151 / 148).
-    const double experts = (double)moe_experts_estimate(q);
-    const double reached = experts * (1.0 - pow(1.0 - 1.0 / experts, (double)q.num_valid));
-    if (bm == 64 && q.block_m < 64 && p.K >= 8192 && reached * ((p.N + 127) / 128) < 150) return false;
+    if (bm == 64 && moe_few_rows_ahead(p, q)) return false;
     if (mode == OUT_F16) launch_moe_tiled_t<OUT_F16>(p, q, bm, st);
     else launch_moe_tiled_t<OUT_BF16>(p, q, bm, st);
     return true;

@@ -739,6 +739,32 @@ def test_fused_moe_a8w8_blocks_put_together(shape):
 
 
 @pytest.mark.parametrize("M,E,N,K,block,kernel", [
+    (8, 8, 16384, 4096, 16, "panel"), (24, 8, 16384, 4096, 16, "panel"), (25, 8, 16384, 4096, 16, "ring"),
+    (64, 8, 16384, 4096, 32, "panel"), (65, 8, 16384, 4096, 32, "ring"), (8, 8, 16384, 4096, 64, "ring"),
+    (2, 8, 16384, 4096, 16, "ring"), (8, 8, 16384, 4160, 16, "ring"), (2, 8, 4096, 6144, 16, "panel"),
+    (2, 8, 4096, 6144, 32, "ring"), (1, 8, 4096, 6144, 64, "ring"), (2, 8, 4096, 4096, 16, "ring")])
+def test_fused_moe_a8w8_blocks_that_keep_the_few_row_kernel(M, E, N, K, block, kernel):
+    """Both sides of the rule that keeps small blocks of wide layers, and few tiles of long rows, on the kernel that streams the
+    weights; the same bits as blocks of 256."""
+    g = torch.Generator(device=DEV).manual_seed(M + K + block)
+    a = torch.randint(-128, 128, (M, K), dtype=torch.int8, device=DEV, generator=g)
+    b = torch.randint(-128, 128, (E, N, K), dtype=torch.int8, device=DEV, generator=g)
+    ar, ac = torch.rand(M, device=DEV, generator=g) * 0.05, torch.rand(E, N, device=DEV, generator=g) * 0.05
+    ids = torch.topk(torch.rand(M, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.rand(M, 2, device=DEV, generator=g)
+
+    def run(block):
+        s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+        c = torch.empty(M, 2, N, dtype=torch.bfloat16, device=DEV)
+        flashnn_amd.fused_moe_a8w8_forward(a, b, c, ar, ac, w, ids, s, e, used, True, 2, block)
+        return c, _lib.last_kernel()
+
+    got, name = run(block)
+    assert name.startswith({"panel": "gemm_a8w8_panel_kernel(moe)", "ring": "gemm_a8w8_ring_kernel(moe"}[kernel]), name
+    assert torch.equal(got, run(256)[0])
+
+
+@pytest.mark.parametrize("M,E,N,K,block,kernel", [
     (2048, 8, 4096, 1024, 128, "(moe)<128,128,4>"),                       # 1.2 rounds of 256-row tiles
     (2048, 8, 4096, 1024, 64, "(moe, blocks together)<128,128,4>"),
     (2048, 8, 4096, 8192, 128, "(moe, blocks together)<256,256,4>"),      # .. of long rows
