@@ -944,8 +944,9 @@ static int group_columns(int bn, int k) { return bn >= 192 && k <= 8192 ? 8 : 4;
 // same memory channels (same box, 0 / 1 slab, us: N=28672 K=8192 M=64 49.5 / 42.9, M=128 58.1 / 49.3, M=256 74.6 / 67.0;
 // N=14784 K=8192 M=100 37.5 / 32.5, M=256 49.0 / 44.2; N=22016 K=4096 M=65 26.3 / 23.7, M=256 37.5 / 35.2; steps of 3 or 11
 // slabs within 2 % of one).  More rows share the pieces through the L2 and gain nothing (M=512: within 1 %; M=2048
-// N=12288 K=4096 86.1 / 87.0), nor do rows with another stride (K = 3584, 5120, 7392, 8896, 17792: within 1 %, 7392 split
-// over two workgroups 33.9 / 34.9).
+// N=12288 K=4096 86.1 / 87.0), nor do rows with another stride (K = 3584, 5120, 7392, 8896, 17792: within 1 %).  With K split
+// over several workgroups the parts of a tile lie apart anyway: 2 to 8 parts over N = 2048 to 8192, K = 8192 to 20480, 65 to 256 rows
+// average 0.94 to 1.00 per number of parts and K on one box, 0.97 to 1.05 on another.
 static int rotation(const A8W8Args& p) { return p.M <= 256 && p.ldb % 4096 == 0 ? 1 : 0; }
 
 template <int BM, int BN, int MODE, bool PAIR = false, int WGM = 2>
@@ -1087,8 +1088,10 @@ static void dispatch_band(A8W8Args& p, hipStream_t st, bool aligned, int force_b
     // N=17792 K=13312 86.0 / 60.0; M=33 alike; M=24: N=24576 K=4096 30.4 / 25.3, N=17792 K=13312 60.9 / 55.9,
     // elsewhere within a few percent, the tiled kernel never behind)
     // (from 9 rows on where the tiled kernel starts its columns apart, see rotation: M=16 N=28672 K=8192 47.0 / 41.8,
-    // N=22016 K=4096 22.8 / 21.1; M=4: 42.9 / 41.4, 20.9 / 20.9)
-    const bool between_rounds = fast && p.M > (rotation(p) ? 8 : 16) && p.M <= 64 && p.N > 16384 && p.N < 32768;
+    // N=22016 K=4096 22.8 / 21.1, K=16384 0.74 to 0.87 over all of these N; M=4: 42.9 / 41.4, 20.9 / 20.9.  At K=4096 only up to
+    // 28672 channels: N=30720 1.02 to 1.04, N=32512 1.03 to 1.05 for 9 to 16 rows, where K=8192 has 0.90 to 0.96)
+    const int apart_from = rotation(p) && (p.N <= 28672 || p.ldb > 4096) ? 8 : 16;
+    const bool between_rounds = fast && p.M > apart_from && p.M <= 64 && p.N > 16384 && p.N < 32768;
     if (force_bm == 0 && !between_rounds && (p.M <= 64 || narrow) && launch_a8w8_skinny(p, MODE, st)) return;
     if (fast && ws.ptr) {
         if (ws.force_kparts > 1) {          // (the entry point has checked tile, parts and workspace size)

@@ -218,6 +218,18 @@ def test_a8w8_between_one_and_two_rounds_of_few_row_workgroups(M, N, K, kernel):
     assert np.array_equal(acc, O.gemm_a8w8_acc(a.numpy(), b.numpy()))
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [(9, 28672, 4096, "ring"), (9, 28688, 4096, "panel"), (16, 32512, 4096, "panel"),
+                                          (17, 32512, 4096, "ring"), (9, 32512, 8192, "ring"), (8, 28672, 4096, "panel")])
+def test_a8w8_few_rows_just_under_two_rounds_of_workgroups(M, N, K, kernel):
+    """9 to 16 rows of K = 4096 over more than 28672 channels stay on the few-row kernel; the same accumulators."""
+    a, b = _rand_i8((M, K), 68), _rand_i8((N, K), 69)
+    ar, ac = torch.rand(M, device=DEV), torch.rand(N, device=DEV)
+    flashnn_amd.GemmA8W8(torch.bfloat16)(a.to(DEV), b.to(DEV), ar, ac)
+    assert _lib.last_kernel().startswith(f"gemm_a8w8_{kernel}_kernel"), _lib.last_kernel()
+    acc = launchers.hip_gemm_a8w8_int32(a.to(DEV), b.to(DEV)).cpu().numpy()
+    assert np.array_equal(acc[:, -512:], O.gemm_a8w8_acc(a.numpy(), b[-512:].numpy()))
+
+
 @pytest.mark.parametrize("M,N,K,tile", [(9, 16640, 4096, "64,128"), (65, 4112, 4096, "64,128"), (256, 12304, 4096, "128,128"),
                                         (250, 22016, 4096, "256,128"), (100, 2048, 8192, None), (257, 4096, 4096, None)])
 def test_a8w8_tile_columns_that_start_apart(M, N, K, tile):
