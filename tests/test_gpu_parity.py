@@ -1079,6 +1079,38 @@ def test_fused_moe_a16w4_per_channel_error_does_not_grow_with_k(K, block):
     assert err ** 2 <= rounding ** 2 * (1 + 1e-3) + added ** 2, (err, rounding, added)
 
 
+@pytest.mark.parametrize("group", [0, 128])
+def test_fused_moe_a16w4_tiles_of_padding_alone_are_left_out(group):
+    """16 rows per expert in blocks of 256: three of four 64-row tiles hold nothing but padding.  The bits of blocks of 64, and,
+    the best of several passes each, at most half as long again (three to four times the tiles before they were left out)."""
+    T, E, N, K = 64, 8, 8192, 4096
+    g = torch.Generator(device=DEV).manual_seed(group)
+    a = torch.randn(T, K, device=DEV, generator=g).half()
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    tables = (E, N) if group == 0 else (E, N, K // group)
+    scale = torch.empty(tables, device=DEV).uniform_(1e-3, 1e-2, generator=g).half()
+    zp = torch.randint(-8, 8, tables, device=DEV, generator=g).half()
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.rand(T, 2, device=DEV, generator=g)
+    out, best = {}, {}
+    for block in (64, 256):
+        routing = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+        c = torch.empty(T, 2, N, dtype=torch.float16, device=DEV)
+        times = []
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(8):
+                flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, *routing, True, 2, block)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        assert _lib.last_kernel().endswith("<4,64,128>"), _lib.last_kernel()
+        out[block], best[block] = c, min(times)
+    assert torch.equal(out[64], out[256])
+    assert best[256] <= 1.5 * best[64], best
+
+
 @pytest.mark.parametrize("kind,E,R,N,K,block,kernel", [
     ("a8w8", 64, 32, 2816, 1024, 32, "gemm_a8w8_ring_kernel(moe, blocks together)<64,128,4>"),
     ("a16w4", 8, 16, 20480, 1024, 16, "gemm_wo_panel_kernel(moe)<4,1,4>")])
