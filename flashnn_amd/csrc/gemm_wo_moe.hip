@@ -354,6 +354,9 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
                     ((uintptr_t)p.act % 16) == 0 && rows * p.lda * 2 < (1LL << 32) && (int64_t)128 * p.ldw < (1LL << 31) &&
                     moe_tiles_estimate(q, 64) * (p.N / 128) < (1LL << 31);
     if (!ok) return false;
+    // The other kernels are preferred only where they take the call: what both refuse (groups of 128 in rows of K / 128 not a
+    // multiple of 8, short rows, tables that are not aligned) would end on the kernel of one thread per output.
+    const bool panel = wo_panel_moe_takes(p, q), others = panel || wo_tile_moe_takes(p, q);
     // Rows of an expert, and what the panel kernel makes of them: it reads the expert's weights once per 16 or 32 rows.  With
     // one such pass and matrices wide enough for its workgroups it stays ahead (same box, groups of 128, panel kernel /
     // 64-row tiles, us - 8 experts N=28672 K=4096: 4 rows per expert 109 / 203, 12 rows 112 / 205, 24 rows 178 / 210, 40 rows 297 /
@@ -361,8 +364,8 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
     // 90, 24 rows 346 / 96; per-channel tables, 8 experts N=4096 K=14336: 12 rows 86 / 102, 24 rows 153 / 100).
     const int64_t experts = moe_experts_estimate(q), mean = (q.num_valid + experts - 1) / experts;
     const int64_t padded = (mean + q.block_m - 1) / q.block_m * q.block_m;
-    if (padded <= 16 && (p.N >= 8192 || p.K >= 8192)) return false;
-    if (padded <= 32 && p.N >= 20480) return false;
+    if (panel && padded <= 16 && (p.N >= 8192 || p.K >= 8192)) return false;
+    if (panel && padded <= 32 && p.N >= 20480) return false;
     // The tile: 128 x 256 where the rows fill it, 64 x 128 (two workgroups per CU) elsewhere.
     // 128 x 256 / 64 x 128 over the three layers above with groups of 128, us: 64 rows per
     // expert 339 / 299 | 270 / 269 | 164 / 135; 100 rows 353 / 395 | 279 / 350 | 170 / 193; 160 rows 621 / 577 | 529 / 498 | 324 / 274;
@@ -372,7 +375,7 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
     auto fits = [&](int bm) { return q.block_m % bm == 0 || bm % q.block_m == 0; };
     const bool rows128 = (mean > 72 && mean < 136) || mean > 208;
     const bool wide = rows128 && fits(128) && p.N % 256 == 0 && moe_tiles_estimate(q, 128) * (p.N / 256) >= 512;
-    if (!wide && (!fits(64) || moe_tiles_estimate(q, 64) * (p.N / 128) < 256)) return false;
+    if (!wide && (!fits(64) || (others && moe_tiles_estimate(q, 64) * (p.N / 128) < 256))) return false;
     auto run = [&](auto adt) {
         constexpr int ADT = decltype(adt)::value;
         if (wide) launch_t<ADT, 128, 256, 2>(p, q, st);

@@ -694,9 +694,7 @@ static bool launch_panel_t(WoArgs& p, hipStream_t st) {
     return true;
 }
 
-template <int ADT>
-static bool launch_panel_moe_t(WoArgs& p, const MoeArgs& q, hipStream_t st) {
-    const int wrows = p.N / 2;
+bool wo_panel_moe_takes(const WoArgs& p, const MoeArgs& q) {
     if (p.N % 32 != 0 || p.K % 32 != 0 || p.K < 8 * 128 || (p.group != 0 && p.group != 128) || q.block_m % 16 != 0 ||
         q.EM % q.block_m != 0 || p.lda % 8 != 0 || p.ldw % 16 != 0 || q.stride_be % 16 != 0 ||
         ((uintptr_t)p.act % 16) != 0 || ((uintptr_t)p.qw % 16) != 0)
@@ -712,6 +710,12 @@ static bool launch_panel_moe_t(WoArgs& p, const MoeArgs& q, hipStream_t st) {
     } else if (q.stride_scale_n != 1 || (p.zp && q.stride_zp_n != 1)) {
         return false;
     }
+    return true;
+}
+
+template <int ADT>
+static void launch_panel_moe_t(WoArgs& p, const MoeArgs& q, hipStream_t st) {
+    const int wrows = p.N / 2;
     int mb_max = q.block_m % 64 == 0 ? 4 : q.block_m % 32 == 0 ? 2 : 1;   // a pass stays within one expert's block
     int rt = 0;
     double best = 0.0;
@@ -753,11 +757,13 @@ static bool launch_panel_moe_t(WoArgs& p, const MoeArgs& q, hipStream_t st) {
     }
 #undef FNN_MOE
 #undef FNN_MOE2
-    return true;
 }
 
 bool launch_wo_panel_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st) {
-    return act_dtype == FNN_F16 ? launch_panel_moe_t<FNN_F16>(p, q, st) : launch_panel_moe_t<FNN_BF16>(p, q, st);
+    if (!wo_panel_moe_takes(p, q)) return false;
+    if (act_dtype == FNN_F16) launch_panel_moe_t<FNN_F16>(p, q, st);
+    else launch_panel_moe_t<FNN_BF16>(p, q, st);
+    return true;
 }
 
 bool launch_wo_panel(WoArgs& p, int wbits, int act_dtype, hipStream_t st) {

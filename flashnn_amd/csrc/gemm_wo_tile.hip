@@ -727,7 +727,7 @@ static bool launch_tile_moe_t(WoArgs& p, const MoeArgs& q, hipStream_t st) {
     return true;
 }
 
-bool launch_wo_tile_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st) {
+bool wo_tile_moe_takes(const WoArgs& p, const MoeArgs& q) {
     const int64_t rows = (q.num_valid + q.top_k - 1) / q.top_k;          // activation rows
     const int G = p.K / 128;
     // group tables: contiguous [expert][channel][group] of one 16-bit type, at most 64 groups
@@ -735,12 +735,14 @@ bool launch_wo_tile_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t 
                                         : p.group == 128 && G <= 64 && is16(p.scale_dtype) && q.stride_scale_k == 1 &&
                                               q.stride_scale_n == G &&
                                               (!p.zp || (p.zp_dtype == p.scale_dtype && q.stride_zp_k == 1 && q.stride_zp_n == G));
-    const bool ok = tables_ok && q.block_m % 128 == 0 && q.EM % q.block_m == 0 && p.N % 128 == 0 &&
-                    p.K % 256 == 0 && p.K >= 512 && p.lda % 8 == 0 && p.ldw % 16 == 0 &&
-                    q.stride_be % 16 == 0 && ((uintptr_t)p.qw % 16) == 0 && ((uintptr_t)p.act % 16) == 0 &&
-                    rows * p.lda * 2 < (1LL << 32) && (int64_t)64 * p.ldw < (1LL << 31) &&
-                    (int64_t)(p.M / 128) * (p.N / 128) < (1LL << 31);
-    if (!ok) return false;
+    return tables_ok && q.block_m % 128 == 0 && q.EM % q.block_m == 0 && p.N % 128 == 0 && p.K % 256 == 0 && p.K >= 512 &&
+           p.lda % 8 == 0 && p.ldw % 16 == 0 && q.stride_be % 16 == 0 && ((uintptr_t)p.qw % 16) == 0 &&
+           ((uintptr_t)p.act % 16) == 0 && rows * p.lda * 2 < (1LL << 32) && (int64_t)64 * p.ldw < (1LL << 31) &&
+           (int64_t)(p.M / 128) * (p.N / 128) < (1LL << 31);
+}
+
+bool launch_wo_tile_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st) {
+    if (!wo_tile_moe_takes(p, q)) return false;
     return act_dtype == FNN_F16 ? launch_tile_moe_t<FNN_F16>(p, q, st) : launch_tile_moe_t<FNN_BF16>(p, q, st);
 }
 

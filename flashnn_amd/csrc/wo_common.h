@@ -285,9 +285,11 @@ bool launch_wo_tile(WoArgs& p, int wbits, int act_dtype, hipStream_t st);
 int wo_tile_count(const WoArgs& p, int wbits);
 // ... its mixture-of-experts form (int4, per-channel tables, blocks of 128 rows or more); false otherwise
 bool launch_wo_tile_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st);
+bool wo_tile_moe_takes(const WoArgs& p, const MoeArgs& q);
 // gemm_wo_moe.hip: int4 mixture of experts with enough rows and tiles to fill the chip; false if the shape does not suit it
 bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st);
 // the int4 per-channel kernel over gathered rows of a mixture of experts; false if the shape does not suit it
 bool launch_wo_panel_moe(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t st);
+bool wo_panel_moe_takes(const WoArgs& p, const MoeArgs& q);
 
 }  // namespace fnn

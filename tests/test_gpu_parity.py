@@ -1111,6 +1111,32 @@ def test_fused_moe_a16w4_tiles_of_padding_alone_are_left_out(group):
     assert best[256] <= 1.5 * best[64], best
 
 
+@pytest.mark.parametrize("T,E,N,K,group,block,kernel", [
+    (16, 8, 28672, 3584, 128, 16, "moe(group tables)"), (16, 8, 28672, 4096, 128, 16, "panel(moe)"),    # 28 and 32 groups
+    (16, 8, 28672, 768, 0, 16, "moe"), (16, 8, 28672, 1024, 0, 16, "panel(moe)"),
+    (40, 8, 20480, 2816, 128, 32, "moe(group tables)"), (2, 4, 1024, 768, 128, 16, "moe(group tables)"),
+    (2, 4, 1024, 1024, 128, 16, "panel(moe)")])
+def test_fused_moe_a16w4_few_rows_that_only_the_tiles_take(T, E, N, K, group, block, kernel):
+    """Small batches are the panel kernel's, but only of the shapes that it takes: not the one-thread-per-output kernel's."""
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    a = torch.randn(T, K, device=DEV, generator=g).half()
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    tables = (E, N) if group == 0 else (E, N, K // group)
+    scale = torch.empty(tables, device=DEV).uniform_(1e-3, 1e-2, generator=g).half()
+    zp = torch.randint(-8, 8, tables, device=DEV, generator=g).half()
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.ones(T, 2, device=DEV)
+    s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+    c = torch.empty(T, 2, N, dtype=torch.float16, device=DEV)
+    flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, False, 2, block)
+    assert _lib.last_kernel().startswith(f"gemm_wo_{kernel.split('(')[0]}_kernel{kernel[len(kernel.split('(')[0]):]}<"), \
+        _lib.last_kernel()
+    for t in range(0, 2 * T, max(1, T // 4)):
+        ex = int(ids.flatten()[t])
+        want = _moe_a16w4_exact(a[t // 2], b[ex], scale[ex], zp[ex])
+        assert float((c.reshape(2 * T, N)[t].double() - want).norm() / want.norm()) < 1e-3
+
+
 @pytest.mark.parametrize("kind,E,R,N,K,block,kernel", [
     ("a8w8", 64, 32, 2816, 1024, 32, "gemm_a8w8_ring_kernel(moe, blocks together)<64,128,4>"),
     ("a16w4", 8, 16, 20480, 1024, 16, "gemm_wo_panel_kernel(moe)<4,1,4>")])
