@@ -22,6 +22,7 @@
 // 8 experts of N=28672 K=4096, groups of 128, bf16, 1024 tokens in blocks of 64: 1266 us on the panel kernel -> 775 (620
 // TFLOP/s); 2048 tokens in blocks of 128 1706 (the fold on 128 x 128 tiles) -> 1415; 64 experts N=2816 K=2048, 64 rows per
 // expert 922 -> 135; per-channel tables, N=4096 K=14336, 250 rows per expert in blocks of 64 1171 -> 370.
+#include <cmath>
 #include <type_traits>
 
 #include "wo_common.h"
@@ -366,6 +367,15 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
     const int64_t padded = (mean + q.block_m - 1) / q.block_m * q.block_m;
     if (panel && padded <= 16 && (p.N >= 8192 || p.K >= 8192)) return false;
     if (panel && padded <= 32 && p.N >= 20480) return false;
+    // Few experts reached: their tiles leave most CUs without one, and the panel kernel's workgroups own a quarter of the channels.
+    // How many tiles that is depends on what else a tile costs, which is K, and on how often the panel kernel reads a block's
+    // weights (once per 16 rows here).  Panel kernel / 64-row tiles, us, per-channel tables: 8 experts N=4096 K=7168, blocks of 16, 1
+    // token 24.7 / 47.8, 2 tokens 25.8 / 48.6, 4 tokens 46.0 / 48.8, 32 tokens level; K=14336, blocks of 64, 1 token 75.8 / 89, 2
+    // tokens 108 / 88; 60 experts N=2816 K=3584, 1 token 21.2 / 26.7, 2 tokens 32.1 / 29.0; K=2048 64 experts N=2816 1 token 26.4 /
+    // 18.3, 128 experts N=1536 20.8 / 18.0.
+    const double e = (double)experts, reached = e * (1.0 - pow(1.0 - 1.0 / e, (double)q.num_valid));
+    const double few = p.K >= 8192 ? 260 : p.K >= 6144 ? 240 : p.K >= 3072 ? 120 : 0;
+    if (panel && padded <= 64 && reached * (p.N / 128) * (padded / 16) < few) return false;
     // The tile: 128 x 256 where the rows fill it, 64 x 128 (two workgroups per CU) elsewhere.
     // 128 x 256 / 64 x 128 over the three layers above with groups of 128, us: 64 rows per
     // expert 339 / 299 | 270 / 269 | 164 / 135; 100 rows 353 / 395 | 279 / 350 | 170 / 193; 160 rows 621 / 577 | 529 / 498 | 324 / 274;

@@ -1115,9 +1115,13 @@ def test_fused_moe_a16w4_tiles_of_padding_alone_are_left_out(group):
     (16, 8, 28672, 3584, 128, 16, "moe(group tables)"), (16, 8, 28672, 4096, 128, 16, "panel(moe)"),    # 28 and 32 groups
     (16, 8, 28672, 768, 0, 16, "moe"), (16, 8, 28672, 1024, 0, 16, "panel(moe)"),
     (40, 8, 20480, 2816, 128, 32, "moe(group tables)"), (2, 4, 1024, 768, 128, 16, "moe(group tables)"),
-    (2, 4, 1024, 1024, 128, 16, "panel(moe)")])
+    (2, 4, 1024, 1024, 128, 16, "panel(moe)"),
+    # few experts reached, both sides of the line
+    (1, 8, 4096, 7168, 0, 16, "panel(moe)"), (2, 8, 4096, 7168, 0, 16, "panel(moe)"), (20, 8, 4096, 7168, 0, 16, "moe"),
+    (1, 64, 2816, 3584, 0, 16, "panel(moe)"), (1, 8, 4096, 8192, 0, 64, "panel(moe)"), (2, 8, 4096, 8192, 0, 64, "moe")])
 def test_fused_moe_a16w4_few_rows_that_only_the_tiles_take(T, E, N, K, group, block, kernel):
-    """Small batches are the panel kernel's, but only of the shapes that it takes: not the one-thread-per-output kernel's."""
+    """Small batches are the panel kernel's where it is ahead, but only of the shapes that it takes: not the
+    one-thread-per-output kernel's."""
     g = torch.Generator(device=DEV).manual_seed(K + N)
     a = torch.randn(T, K, device=DEV, generator=g).half()
     b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
