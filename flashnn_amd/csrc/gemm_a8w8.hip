@@ -1191,14 +1191,6 @@ static void launch_mfma_moe(A8W8Args& p, const MoeArgs& q, hipStream_t st) {
 // Tile heights that the block size allows: the tile is a part of a block, or whole blocks make up the tile.
 static bool moe_tile_fits(const MoeArgs& q, int bm) { return q.block_m >= 16 && (q.block_m % bm == 0 || bm % q.block_m == 0); }
 
-// Rounds of tiles of bm x bm that a call makes with per_round of them at a time, the rows of an expert taken as spread round
-// their mean the way an even random routing spreads them.
-static double moe_rounds(const A8W8Args& p, const MoeArgs& q, int bm, int per_round) {
-    const double experts = (double)moe_experts_estimate(q), mean = (double)q.num_valid / experts, off = 1.2 * sqrt(mean);
-    const double tall = (ceil((mean - off) / bm) + ceil(mean / bm) + ceil((mean + off) / bm)) / 3.0;
-    return experts * tall * ((p.N + bm - 1) / bm) / per_round;
-}
-
 // The height of the tiles.  Blocks of a multiple of 128 rows keep tiles of at least 128, of 256 rows those of 256 (what the
 // caller sorted for).  Else by the mean number of routed rows per expert (estimated, moe_experts_estimate), where the
 // tiles fill the chip; with fewer than one round of the taller tiles, 64 rows.  Measured over
@@ -1221,8 +1213,8 @@ static int moe_tile_rows(const A8W8Args& p, const MoeArgs& q) {
     int bm = mean <= 56 ? 64 : mean < 144 ? 128 : 256;
     while (bm > least && (!moe_tile_fits(q, bm) || moe_tiles_estimate(q, bm) * ((p.N + bm - 1) / bm) < 256)) bm /= 2;
     if (bm == 256 && least < 256 && p.K < 8192) {
-        const double whole = ceil(moe_rounds(p, q, 256, 256) - 0.05);
-        if (whole > 1.0 && (least == 128 ? 1.66 : 1.5) * whole > moe_rounds(p, q, 128, 512) + 0.25) bm = 128;
+        const double whole = ceil(moe_rounds(q, p.N, 256, 256, 256) - 0.05);
+        if (whole > 1.0 && (least == 128 ? 1.66 : 1.5) * whole > moe_rounds(q, p.N, 128, 128, 512) + 0.25) bm = 128;
     }
     return bm > least ? bm : least;
 }

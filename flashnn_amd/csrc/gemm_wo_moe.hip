@@ -376,16 +376,25 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
     const double e = (double)experts, reached = e * (1.0 - pow(1.0 - 1.0 / e, (double)q.num_valid));
     const double few = p.K >= 8192 ? 260 : p.K >= 6144 ? 240 : p.K >= 3072 ? 120 : 0;
     if (panel && padded <= 64 && reached * (p.N / 128) * (padded / 16) < few) return false;
+    // with fewer narrow tiles than CUs the workgroups of the other kernels are no worse off
+    if (others && moe_tiles_estimate(q, 64) * (p.N / 128) < 256) return false;
     // The tile: 128 x 256 where the rows fill it, 64 x 128 (two workgroups per CU) elsewhere.
     // 128 x 256 / 64 x 128 over the three layers above with groups of 128, us: 64 rows per
     // expert 339 / 299 | 270 / 269 | 164 / 135; 100 rows 353 / 395 | 279 / 350 | 170 / 193; 160 rows 621 / 577 | 529 / 498 | 324 / 274;
-    // 256 rows 775 / 853 | 690 / 714 | 396 / 395; 512 rows 1415 / 1567 | 1225 / 1326.  N=4096 K=14336, fewer than 512 wide tiles: 100 rows
-    // 207 / 148, 256 rows 417 / 370; 512 rows (640 wide tiles) 637 / 649.
-    // With fewer narrow tiles than CUs the workgroups of the other kernels are no worse off.
+    // 256 rows 775 / 853 | 690 / 714 | 396 / 395; 512 rows 1415 / 1567 | 1225 / 1326.  N=4096 K=14336, per-channel tables, fewer than
+    // 512 wide tiles: 100 rows 207 / 148, 250 rows 421 / 378.
+    // Blocks of 128 rows and more, which gemm_wo_tile_kernel's 128 x 128 tiles had, by rounds: the wide tiles run one to a CU in whole
+    // rounds, of the narrow ones what is left over of a round runs beside the end of the one before, and a round of the first takes
+    // about 1.55 times one of the second (128 x 128 / 128 x 256 / 64 x 128, per-channel tables: N=4096 K=14336, 188 rows, 1.0 rounds of wide
+    // tiles 272 / 245 / 290, 512 rows, 2.2 rounds 646 / 683 / 667; 4 experts N=16384 K=5120, 128 rows, 1.4 rounds 152 / 171 / 145).
     auto fits = [&](int bm) { return q.block_m % bm == 0 || bm % q.block_m == 0; };
-    const bool rows128 = (mean > 72 && mean < 136) || mean > 208;
-    const bool wide = rows128 && fits(128) && p.N % 256 == 0 && moe_tiles_estimate(q, 128) * (p.N / 256) >= 512;
-    if (!wide && (!fits(64) || (others && moe_tiles_estimate(q, 64) * (p.N / 128) < 256))) return false;
+    bool wide = (mean > 72 && mean < 136) || mean > 208;
+    if (q.block_m % 128 == 0)
+        wide = moe_rounds(q, p.N, 64, 128, 512) + 0.25 > 1.55 * ceil(moe_rounds(q, p.N, 128, 256, 256) - 0.05);
+    else
+        wide = wide && moe_tiles_estimate(q, 128) * (p.N / 256) >= 512;
+    wide = wide && fits(128) && p.N % 256 == 0;
+    if (!wide && !fits(64)) return false;
     auto run = [&](auto adt) {
         constexpr int ADT = decltype(adt)::value;
         if (wide) launch_t<ADT, 128, 256, 2>(p, q, st);

@@ -1,6 +1,8 @@
 // Gather/scatter description shared by the mixture-of-experts forms of the few-row GEMM kernels.
 #pragma once
 
+#include <cmath>
+
 #include "fnn_common.h"
 
 namespace fnn {
@@ -104,6 +106,13 @@ inline int64_t moe_tiles_estimate(const MoeArgs& q, int bm) {
     if (q.block_m >= bm) return blocks * (q.block_m / bm);
     const int64_t t = (q.num_valid + bm - 1) / bm + moe_experts_estimate(q);
     return t < blocks ? t : blocks;
+}
+// ... and the rounds of tiles of bm rows x bn of n channels that a call makes with per_round of them at a time, the rows of an
+// expert taken as spread round their mean the way an even random routing spreads them
+inline double moe_rounds(const MoeArgs& q, int n, int bm, int bn, int per_round) {
+    const double experts = (double)moe_experts_estimate(q), mean = (double)q.num_valid / experts, off = 1.2 * sqrt(mean);
+    const double tall = (ceil((mean - off) / bm) + ceil(mean / bm) + ceil((mean + off) / bm)) / 3.0;
+    return experts * tall * ((n + bn - 1) / bn) / per_round;
 }
 
 }  // namespace fnn

@@ -1079,6 +1079,29 @@ def test_fused_moe_a16w4_per_channel_error_does_not_grow_with_k(K, block):
     assert err ** 2 <= rounding ** 2 * (1 + 1e-3) + added ** 2, (err, rounding, added)
 
 
+@pytest.mark.parametrize("T,N,block,tile", [
+    (700, 4096, 128, "128,256"), (560, 8192, 128, "64,128"),          # 1.0 and 1.7 rounds of wide tiles
+    (700, 4096, 64, "64,128"), (2048, 8192, 16, "128,256"), (2048, 8192, 128, "128,256")])
+def test_fused_moe_a16w4_tile_by_rounds(T, N, block, tile):
+    """Blocks of 128: wide tiles where they make whole rounds, narrow ones for a little more (rows against 64 bits)."""
+    E, K = 8, 1024
+    g = torch.Generator(device=DEV).manual_seed(T + N)
+    a = torch.randn(T, K, device=DEV, generator=g).half()
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    scale = torch.empty(E, N, K // 128, device=DEV).uniform_(1e-3, 1e-2, generator=g).half()
+    zp = torch.randint(-8, 8, (E, N, K // 128), device=DEV, generator=g).half()
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.rand(T, 2, device=DEV, generator=g)
+    s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+    c = torch.empty(T, 2, N, dtype=torch.float16, device=DEV)
+    flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, False, 2, block)
+    assert _lib.last_kernel() == f"gemm_wo_moe_kernel(group tables)<4,{tile}>", _lib.last_kernel()
+    for t in range(0, 2 * T, T // 3):
+        ex = int(ids.flatten()[t])
+        want = _moe_a16w4_exact(a[t // 2], b[ex], scale[ex], zp[ex])
+        assert float((c.reshape(2 * T, N)[t].double() - want).norm() / want.norm()) < 1e-3
+
+
 @pytest.mark.parametrize("group", [0, 128])
 def test_fused_moe_a16w4_tiles_of_padding_alone_are_left_out(group):
     """16 rows per expert in blocks of 256: three of four 64-row tiles hold nothing but padding.  The bits of blocks of 64, and,
