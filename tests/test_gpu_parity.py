@@ -957,6 +957,56 @@ def test_fused_moe_a16w4_many_rows_close(shape, group, zp_kind, act_ty):
             assert (want == 3.0).all(axis=1).any() and np.array_equal((got == 3.0).all(axis=1), (want == 3.0).all(axis=1))
 
 
+@pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K", [(5, 2048), (4100, 4096), (2050, 8192)])
+def test_norm_rows_with_infinities_nan_and_in_place(hip_lib, M, K, ty):
+    """Rows with an infinity, a NaN, the largest values and nothing but zeros between ordinary ones: the bits of the
+    one-workgroup-per-row kernel.  And the output over the input, where a workgroup requests its next row before it writes."""
+    g = torch.Generator().manual_seed(M + K)
+    x = (torch.randn(M, K, generator=g) * 3).to(ty)
+    for row, value in ((0, float("inf")), (1, float("nan")), (2, float("-inf")), (3, torch.finfo(ty).max)):
+        x[row::max(M - 1, 5), K // 3] = value
+    x[4] = 0
+    x = x.to(DEV)
+    w = torch.empty(K).uniform_(0.5, 1.5, generator=g).to(ty).to(DEV)
+    b = torch.empty(K).uniform_(-0.5, 0.5, generator=g).to(ty).to(DEV)
+    bits = lambda t: t.view(torch.int16) if t.element_size() == 2 else t
+    for op, kernel in ((lambda w, b: (launchers.hip_rmsnorm_forward(x, w, 1e-6),), 0),
+                       (lambda w, b: (launchers.hip_layer_norm_forward(x, w, b, 1e-5),), 1),
+                       (lambda w, b: launchers.hip_layer_norm_dquant_forward(x, w, b, 1e-5), 2)):
+        got = op(w, b)
+        assert _lib.last_kernel().startswith(f"norm_rows_kernel<{kernel},"), _lib.last_kernel()
+        for u, v in zip(got, op(w.float(), b.float())):
+            assert torch.equal(bits(u), bits(v))
+    code, st = _lib.dtype_code(ty), _lib.current_stream(torch.device(DEV))
+    for op, ref in ((lambda t: hip_lib.fnn_rmsnorm(t.data_ptr(), t.data_ptr(), w.data_ptr(), 1e-6, M, K, K, K, code, code, st),
+                     launchers.hip_rmsnorm_forward(x, w, 1e-6)),
+                    (lambda t: hip_lib.fnn_layernorm(t.data_ptr(), t.data_ptr(), w.data_ptr(), b.data_ptr(), 1e-5, M, K, K, K, code,
+                                                     code, st), launchers.hip_layer_norm_forward(x, w, b, 1e-5))):
+        t = x.clone()
+        assert op(t) == 0, hip_lib.fnn_last_error()
+        assert _lib.last_kernel().startswith("norm_rows_kernel<"), _lib.last_kernel()
+        assert torch.equal(bits(t), bits(ref))
+
+
+@pytest.mark.parametrize("row", [2048, 22528])
+@pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
+def test_dynamic_quantize_every_16_bit_quotient(ty, row):
+    """Rows whose largest value is 127, so that the scale is 1 and the quotients are the inputs: every 16-bit value of at most
+    127, ties among them, is rounded to the nearest integer, halves to the even one."""
+    top = int(torch.tensor([127.0], dtype=ty).view(torch.int16))
+    t = torch.arange(top + 1, dtype=torch.int32).to(torch.int16).view(ty)
+    t = torch.cat([t, -t])
+    rows = -(-t.numel() // (row - 8))
+    x = torch.full((rows, row), 127.0, dtype=ty)
+    padded = torch.full((rows * (row - 8),), 127.0, dtype=ty)
+    padded[:t.numel()] = t
+    x[:, :row - 8] = padded.reshape(rows, row - 8)
+    q, s = flashnn_amd.DynamicQuantize()(x.to(DEV))
+    assert bool((s == 1).all())
+    assert torch.equal(q.cpu().float(), torch.round(x.float()))
+
+
 @pytest.mark.parametrize("gb_ty", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K", [(1, 2048), (2047, 2056), (2049, 4096), (4100, 2568), (3, 8192)])
@@ -989,6 +1039,20 @@ def _moe_a16w4_exact(a, packed, scale, zp):
     return ((nib * scale.double().reshape(N, G, 1)).reshape(N, K) * a.double()).sum(1)
 
 
+def _moe_a16w4_worst(got, want, a, scale, weight):
+    """The largest of a row's errors over what is allowed, 1 and less being in order.  Value by value: one rounding to 16 bits and
+    the fp32 sums of 128 products a * (c + q), c = 1032 or 136, each at most 128 2^-24 of their magnitudes before c and the zero
+    point come off.  That is a worst case and several per cent of a small result, so the row as a whole must also lie
+    within 1e-3 (bf16: 5e-3) of its 2-norm, about five (three) times what the output's rounding alone gives."""
+    fp16 = got.dtype == torch.float16
+    K, N = a.shape[0], scale.shape[0]
+    slabs = a.double().abs().reshape(K // 128, 128).sum(1) * (1048.0 if fp16 else 152.0)
+    mags = (slabs * scale.double().reshape(N, -1)).sum(1)          # (per-channel tables: one scale for all slabs)
+    bound = want.abs() * (2.0 ** -11 if fp16 else 2.0 ** -8) * 1.01 + mags * 2.0 ** -24 * 128 * weight + 1e-7
+    err = (got.double() - want).abs()
+    return max(float((err / bound).max()), float(err.norm() / want.norm()) / (1e-3 if fp16 else 5e-3))
+
+
 @pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("group,with_zp", [(0, True), (0, False), (128, True), (128, False)])
 @pytest.mark.parametrize("shape", [
@@ -997,7 +1061,7 @@ def _moe_a16w4_exact(a, packed, scale, zp):
     (400, 4, 16384, 4096, 1, 64, "128,256"), (1300, 5, 5376, 512, 2, 64, "128,256"), (900, 2, 19200, 1280, 1, 128, "128,256")])
 def test_fused_moe_a16w4_blocks_put_together(shape, group, with_zp, act_ty):
     """The tiled kernel over blocks of one expert put together, against float64 products of the same integers, activations and
-    tables: fp32 sums of K products (K 2^-24 of their magnitudes at most) and one rounding to 16 bits.  The bits do not hang on
+    tables (_moe_a16w4_worst).  The bits do not hang on
     the order of the blocks (shuffled: runs of one block, more tiles than the grid was sized for), on strided operands or on a
     list cut in the middle, whose other rows keep their value."""
     M, E, N, K, top_k, BM, tile = shape
@@ -1022,19 +1086,10 @@ def test_fused_moe_a16w4_blocks_put_together(shape, group, with_zp, act_ty):
     a = abuf[:, :K].contiguous()
     got = run(a, s, e, used)
     for t in range(0, M * top_k, max(1, M * top_k // 40)):
-        ex = int(ids.flatten()[t])
-        nib = torch.stack([(b[ex] << 4) >> 4, b[ex] >> 4], 1).reshape(N, K).double()
-        G = 1 if group == 0 else K // group
-        z = zp[ex].double().reshape(N, G, 1) if with_zp else 0.0
-        terms = (nib.reshape(N, G, K // G) - z) * scale[ex].double().reshape(N, G, 1) * a[t // top_k].double().reshape(1, G, K // G)
-        want = terms.sum((1, 2)) * w.flatten()[t].double()
-        # the sums run over a * (c + q), c = 1032 or 136, before c and the zero point are taken off
-        off = 1048.0 if act_ty == torch.float16 else 152.0
-        mags = (a[t // top_k].double().abs().reshape(1, G, K // G).sum(2) * off * scale[ex].double().reshape(N, G)).sum(1)
-        bound = want.abs() * (2.0 ** -11 if act_ty == torch.float16 else 2.0 ** -8) * 1.01 + mags * 2.0 ** -24 * (K // G) * \
-            w.flatten()[t].double() + 1e-7
-        err = (got.reshape(M * top_k, N)[t].double() - want).abs()
-        assert bool((err <= bound).all()), (t, float((err / bound).max()))
+        ex, tw = int(ids.flatten()[t]), w.flatten()[t].double()
+        want = _moe_a16w4_exact(a[t // top_k], b[ex], scale[ex], zp[ex] if with_zp else None) * tw
+        worst = _moe_a16w4_worst(got.reshape(M * top_k, N)[t], want, a[t // top_k], scale[ex], tw)
+        assert worst <= 1.0, (t, worst)
     assert torch.equal(run(abuf[:, :K], s, e, used, pad=9), got)
     order = torch.randperm(int(used[0]) // BM)
     s2, e2 = s.clone(), e.clone()

@@ -271,7 +271,8 @@ def test_empty_calls_need_no_addresses(hip_lib):
 
 @pytest.mark.parametrize("ty", [torch.float16, torch.bfloat16])
 def test_biased_byte_needs_no_rounding_of_its_own(ty):
-    """Every 16-bit quotient: 128 added in fp32 and rounded to nearest even is the rounded quotient plus 128."""
+    """The arithmetic behind the paired byte conversion, in torch: for every 16-bit quotient, 128 added in fp32 and rounded to
+    nearest even is the rounded quotient plus 128.  (The kernels: test_dynamic_quantize_every_16_bit_quotient.)"""
     t = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(ty).float()
     t = t[torch.isfinite(t) & (t.abs() <= 4096)]
     assert torch.equal(torch.round(t + 128.0), torch.round(t) + 128.0)

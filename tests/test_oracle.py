@@ -601,3 +601,30 @@ def test_one_step_dequantisation_equals_the_two_roundings():
     two = (q.bfloat16() - zp_bad) * s1
     one = ((q.double() - zp_bad.double()) * s1.double()).float().bfloat16()
     assert not torch.equal(one[:, 0], two[:, 0]) and not torch.equal(one[:, 1], two[:, 1])
+
+
+@pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("group", [0, 128])
+@pytest.mark.parametrize("K", [512, 4096])
+def test_moe_a16w4_row_check_finds_planted_mistakes(K, group, act_ty):
+    """What the GPU tests hold the tiled A16W4 kernel to: the exact row, rounded, passes; zeros, a neighbour's zero points, a
+    neighbour's scales, a slab of K left out and a nibble pair taken the wrong way round do not."""
+    from test_gpu_parity import _moe_a16w4_exact, _moe_a16w4_worst
+    N = 256
+    g = torch.Generator().manual_seed(K + group)
+    a = torch.randn(K, generator=g).to(act_ty)
+    packed = torch.randint(-128, 128, (N // 2, K), dtype=torch.int8, generator=g)
+    tables = (N,) if group == 0 else (N, K // group)
+    scale = torch.empty(tables).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
+    zp = torch.empty(tables).uniform_(-8, 8, generator=g).to(act_ty)
+    want = _moe_a16w4_exact(a, packed, scale, zp) * 0.5
+    worst = lambda row: _moe_a16w4_worst((row * 0.5).to(act_ty), want, a, scale, 0.5)
+    assert worst(want * 2) <= 1.0
+    assert worst(want * 0) > 1.0
+    assert worst(_moe_a16w4_exact(a, packed, scale, zp.roll(1, 0))) > 1.0
+    assert worst(_moe_a16w4_exact(a, packed, scale.roll(1, 0), zp)) > 1.0
+    without = a.clone()
+    without[256:384] = 0
+    assert worst(_moe_a16w4_exact(without, packed, scale, zp)) > 1.0
+    other = ((packed << 4) & -16) | ((packed >> 4) & 15)
+    assert worst(_moe_a16w4_exact(a, other, scale, zp)) > 1.0
