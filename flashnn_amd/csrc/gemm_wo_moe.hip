@@ -18,7 +18,8 @@
 // (7.7 ns against 7.4 alone), three cost 9.5 ns and four 12.8; a slab of the 128 x 256 tile has 80 MFMAs and about 310 of
 // them per wave (conversion 128, fold 128).  Wave tiles of 128 x 32 with the conversion a slab ahead (2.1 per MFMA, but half as
 // many MFMAs again against ones) measured the same (773 us below), one wave per SIMD with 128 x 64 was slower (1113: the
-// accumulators move between the register files).
+// accumulators move between the register files).  The 128 x 256 tile with group tables needs more than its 256 registers: 15 (bf16
+// tables) and 29 (fp16) are spilled, to 64 and 112 bytes a lane; per-channel tables (243 registers) and the 64 x 128 tile spill none.
 // 8 experts of N=28672 K=4096, groups of 128, bf16, 1024 tokens in blocks of 64: 1266 us on the panel kernel -> 775 (620
 // TFLOP/s); 2048 tokens in blocks of 128 1706 (the fold on 128 x 128 tiles) -> 1415; 64 experts N=2816 K=2048, 64 rows per
 // expert 922 -> 135; per-channel tables, N=4096 K=14336, 250 rows per expert in blocks of 64 1171 -> 370.
@@ -32,7 +33,9 @@ namespace fnn {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 
-constexpr int kGroups = 32;        // K / 128 at most, where there are group tables
+// K / 128 at most, where there are group tables: they lie in LDS whole, 33 KB for 32 groups of 256 channels beside 112 KB of
+// stages, and 64 groups do not fit the 160 KB.  Longer rows (K = 4224 to 8192) stay on gemm_wo_tile_kernel and the panel kernel.
+constexpr int kGroups = 32;
 
 // One tile: rows m0 .. row_end - 1 (at most BM) of the sorted list, channels n0 .. n0 + BN - 1 of one expert.
 template <int ADT, bool GROUPS, int SDT, int BM, int BN, int WGM>

@@ -11,9 +11,9 @@ namespace fnn {
 
 constexpr int kRowThreads = 256;
 
-// Block reductions over the four waves of a workgroup.  `red` serves ONE reduction per kernel (nothing
-// guards it against being written again while a slow wave still reads it): every kernel here reduces once
-// through each of its arrays.
+// Block reductions over the four waves of a workgroup.  A slow wave may still read `red` when a fast one has left: the same
+// array may be written again only behind another barrier that every wave has crossed since.  Kernels of one row reduce once
+// through each of their arrays; the row-walking norms take two by turns, so that the next row's barrier lies between.
 __device__ __forceinline__ float block_max(float v, float* red) {
     v = wave_max(v);
     const int w = threadIdx.x >> 6;

@@ -156,8 +156,10 @@ __global__ __launch_bounds__(kRowThreads) void norm_vec_kernel(const NormArgs p)
 // A workgroup walks several rows.  The next row is requested before this one is worked on, and gamma and beta (16-bit) stay in
 // registers as they came, so a row costs its own loads only and they are on their way during the arithmetic of the row
 // before.  That arithmetic is what bounds it with quantisation (about 20 vector instructions a value: four for the fp64
-// moments, nine to normalise, six to quantise; 4001 x 8192 in 29.8 us against 16 us of memory time at 6 TB/s), so values are
-// rounded in pairs.
+// moments, nine to normalise, six to quantise; 4001 x 8192 in 29.8 us with rotating inputs under a captured graph, 25.5 a call in a
+// stream of calls, against 16 us of memory time at 6 TB/s), so values are rounded in pairs.  It also bounds how many hide it:
+// rows of 4097 to 8192 values take 146 to 152 registers (rmsnorm 110), three workgroups a CU, so 768 of up to 2048 are resident and a
+// call of 4001 rows gives a workgroup two.
 template <int DT, int NV, int OP, int GB>
 __global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const NormArgs p, const int rows) {
     __shared__ double redd[2][8];       // (by turns: a slow wave may still read what the row before left)

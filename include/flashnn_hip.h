@@ -345,9 +345,10 @@ int fnn_gemm_a8w8_i32_tiled(int32_t* acc, const void* a, const void* b, int64_t 
  * are left untouched.  sorted_token_ids [EM], expert_ids and num_tokens_post_padded [1] are int32 device
  * arrays.  K >= 1024, K % 32 == 0, EM % block_m == 0, 16-byte aligned rows and block_m 16, 32, 64 or a multiple of 64:
  * MFMA tiles of 64, 128 or 256 sorted rows.  A tile is a part of one block or, where blocks are smaller, several
- * consecutive blocks of one expert, so block_m decides the padding and not the speed.  A few rows over few channels,
- * and other multiples of 16, take a weight-streaming kernel (N % 16 == 0); anything else a slow guarded kernel.  The same
- * arithmetic and the same bits everywhere.
+ * consecutive blocks of one expert, so block_m decides the padding and little of the speed (lists of many hundred blocks take up to a
+ * quarter longer in blocks of 16 than of 64: every tile searches the list).  Blocks of 16 and 32 with a few rows per expert, over
+ * few channels of long rows or wide layers whose rows lie a multiple of 4 KiB apart, and other multiples of 16, take a
+ * weight-streaming kernel (N % 16 == 0); anything else a slow guarded kernel.  The same arithmetic and the same bits everywhere.
  */
 int fnn_fused_moe_a8w8(void* c, const void* a, const void* b, const void* alpha_row,
                        const void* alpha_col, const void* topk_weights,
@@ -381,7 +382,7 @@ int fnn_fused_moe_a8w8(void* c, const void* a, const void* b, const void* alpha_
  * either group = 0 with floating zero points or group = 128 with contiguous tables of one 16-bit type (zero points in the
  * scales' type) the call runs tiled MFMA kernels over the sorted rows.  K <= 4096 for group = 128, block_m 16, 32, 64 or a
  * multiple of 64: a tile is a part of one block or several consecutive blocks of one expert (128 rows x 256 channels or 64 x 128),
- * so block_m decides the padding and not the speed.  Few tiles, or K <= 8192: block_m a multiple of 128, tiles of 128 or 256 rows
+ * so block_m decides the padding and little of the speed.  Few tiles, or K <= 8192: block_m a multiple of 128, tiles of 128 or 256 rows
  * x 128 channels.
  */
 int fnn_fused_moe_a16w4(void* c, const void* a, const void* b, const void* scale_b,
