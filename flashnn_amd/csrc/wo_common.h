@@ -2,6 +2,8 @@
 // integer -> fp16/bf16 conversions that run on exponent tricks.
 #pragma once
 
+#include <type_traits>
+
 #include "fnn_common.h"
 #include "moe_common.h"
 
@@ -34,6 +36,19 @@ inline int group_shift(int group) {
     for (int s = 0; s < 16; ++s)
         if (group == (128 << s)) return s;
     return -1;
+}
+
+// Address of a __shared__ object for copy_to_lds_16
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+// Every lane copies 16 bytes from base + off (base the same for the whole wave) to LDS, the wave's kilobyte one lane behind the
+// other from `to` on.  Written as asm because the compiler does not know which stage of a ring a copy fills where the stage is
+// chosen at run time, and then waits for every copy in flight before each LDS read: here the caller waits
+// (s_waitcnt vmcnt) and nobody else.  No register is written.
+__device__ __forceinline__ void copy_to_lds_16(const char* base, uint32_t off, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(__builtin_amdgcn_readfirstlane(to)), "v"(off), "s"(base) : "memory", "m0");
 }
 
 constexpr int kWoWaves = 8;
@@ -264,6 +279,30 @@ __device__ __forceinline__ void convert_w4_nat_f16_2off(const v4u w, v4u& e0, v4
         o[2 * q] = (y & m1) ^ c1;
         e[2 * q + 1] = (y2 & m0) ^ c0;
         o[2 * q + 1] = (y2 & m1) ^ c1;
+    }
+    e0 = v4u{e[0], e[1], e[2], e[3]};
+    e1 = v4u{e[4], e[5], e[6], e[7]};
+    o0 = v4u{o[0], o[1], o[2], o[3]};
+    o1 = v4u{o[4], o[5], o[6], o[7]};
+}
+
+// The same as plain whole numbers u = v + 8 (0 .. 15): a byte that holds no more than a nibble is, read as an fp8 number
+// (e4m3: 2^-9 a step up to 15), u * 2^-9, and the conversion instruction multiplies by 2^9.  14 vector instructions per 16
+// weights against 16 of convert_w4_nat, and sums of products that carry 8 times the activation sum, not 136 or 1032 times.
+template <int ADT>
+__device__ __forceinline__ void convert_w4_u(const v4u w, v4u& e0, v4u& e1, v4u& o0, v4u& o1) {
+    auto two = [](uint32_t x, auto hi) {
+        if constexpr (ADT == FNN_F16) return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 512.f, decltype(hi)::value));
+        else return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 512.f, decltype(hi)::value));
+    };
+    uint32_t e[8], o[8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t lo = (w[q] & 0x0F0F0F0Fu) ^ 0x08080808u, hi = ((w[q] >> 4) & 0x0F0F0F0Fu) ^ 0x08080808u;
+        e[2 * q] = two(lo, std::false_type{});
+        e[2 * q + 1] = two(lo, std::true_type{});
+        o[2 * q] = two(hi, std::false_type{});
+        o[2 * q + 1] = two(hi, std::true_type{});
     }
     e0 = v4u{e[0], e[1], e[2], e[3]};
     e1 = v4u{e[4], e[5], e[6], e[7]};
