@@ -1,7 +1,7 @@
 // Weight-only GEMM for 9 .. a few hundred activation rows ("panel" kernel, gfx950).
 //
 // The weights are still read exactly once per pass and go straight from global memory into the
-// MFMA "A" operand; what changes against the decode kernels is the activation side.  With 16..64
+// MFMA operands; what changes against the decode kernels is the activation side.  With 16..64
 // activation rows every weight tile needs M*K*2 bytes of activations, too much to pull through
 // the vector memory path once per 16 weight rows.  Here a workgroup owns 64 weight rows (four
 // waves, 16 rows each) and the four waves share each 128-k slab of the activation panel through
@@ -14,14 +14,14 @@
 //   * weights: two 16-byte loads per lane and slab, kept 4 slabs ahead in registers and fetched
 //     as full 128-byte lines (8 rows per load); a wave-private LDS staging area reshapes them into
 //     the MFMA operand layout; the refill of a register is issued right after its last use;
-//   * group scales and zero points (group == 128): one 16-byte load each per lane and slab,
-//     4 slabs ahead, folded into the running output at the end of each slab:
+//   * group scales and zero points (group == 128): one load each per lane and slab, 4 slabs ahead, folded
+//     into the running output slab by slab:
 //         out += s * (acc - (c + zp) * sum_k a_k),
-//     c being the constant the exponent-trick conversion adds, sum_k a_k coming from an MFMA
-//     against ones;
+//     c being the constant the conversion adds (8 for int4 weights scaled in fp32: ROWS below), sum_k a_k coming
+//     from an MFMA against ones;
 //   * all loads of an iteration are issued in a fixed order, so "slab j has landed" is one
 //     s_waitcnt vmcnt(X) with a compile-time X, followed by a bare s_barrier;
-//   * the K parts are added through LDS in a fixed order, then bias, rounding, 16-byte stores.
+//   * the K parts are added through LDS in a fixed order, then bias, rounding, stores.
 //
 // Reference semantics: flashnn/quant_gemm.py:148-206.
 #include <type_traits>
@@ -71,6 +71,15 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
     typedef MfmaT<ADT> MT;
     constexpr int NH = WBITS == 4 ? 2 : 1;      // channels per weight row
     constexpr int NCL = 4 * NH;                 // consecutive channels per lane
+    // int4 weights scaled in fp32: the activations are the first MFMA operand, so that a lane's sums are of one weight row (two
+    // channels) and a slab's fold takes two scales and two zero points per lane instead of eight of each; the weights enter as
+    // u = v + 8, 0 .. 15.  16 rows a pass: over 85 calls of seven matrices 4.5 % less time; 32 rows a
+    // pass 7 % less with per-channel tables, but 3 to 5 % more with groups over K=8192 (34.5 -> 36.5), which stay as they were.
+    constexpr bool ROWS = WBITS == 4 && !REFQ && !(G128 && MB == 2);
+    // ... and with 64 rows a pass the four waves of a K part, which multiply the same activations, sum up the rows of one block each
+    // and hand the sums on through LDS: read a slab later, so that no barrier is added (53.5 us with MFMAs against ones for every block
+    // in every wave, 49.8 with shared sums; with 32 rows a pass the exchange costs more than the four MFMAs that it saves)
+    constexpr bool DIST = ROWS && GSUB == 1 && MB == 4 && RT == 4;
     constexpr float c_off = WBITS == 4 ? (ADT == FNN_F16 ? 1024.f + 8.f : 128.f + 8.f)
                                        : (ADT == FNN_F16 ? 1024.f + 128.f : 128.f);
     constexpr int SLAB = MB * 16 * 256;         // bytes of one activation slab: 16*MB rows x 128 k
@@ -191,11 +200,11 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
         for (int h = 0; h < 2; ++h) rd[s][h] = ks * SLAB + li * 256 + (((s * 8 + lg * 2 + h) ^ li) << 4);
 
     // ---- group tables: NCL consecutive channels per lane
-    typedef typename std::conditional<NH == 2, v4u, v2u>::type tab_t;
-    const int n0 = NH * (row0 + 4 * lg);
+    typedef typename std::conditional<ROWS, uint32_t, typename std::conditional<NH == 2, v4u, v2u>::type>::type tab_t;
+    const int n0 = NH * (row0 + (ROWS ? li : 4 * lg));      // first of the lane's channels
     const uint16_t* sptr = (const uint16_t*)p.scale + NH * row0;             // scalar
     const uint16_t* zptr = (p.zp ? (const uint16_t*)p.zp : (const uint16_t*)p.scale) + NH * row0;
-    const uint32_t tab_off = NH * 4 * lg * 2;                                                        // bytes
+    const uint32_t tab_off = ROWS ? 4 * li : NH * 4 * lg * 2;                                                        // bytes
     const bool has_zp = p.zp != nullptr;
     // without zero points the second table load reads the scales again and is multiplied away
     const float zmul = has_zp ? 1.f : 0.f;
@@ -257,32 +266,175 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
     constexpr int CHW = RT * 16 * NH;           // channels of the workgroup
     constexpr int TABG_MAX = 64;                // groups the LDS tables hold (K <= 8192)
     __shared__ __attribute__((aligned(16))) uint16_t tabs[TABLDS ? 2 * TABG_MAX * CHW : 8];
-    const int chl = NH * (rt * 16 + 4 * lg);    // the lane's first channel within the workgroup
+    const int chl = NH * (rt * 16 + (ROWS ? li : 4 * lg));    // the lane's first channel within the workgroup
     auto lds_tab = [&](int which, int jj) -> tab_t {
         const int kg = sl0 + min(jj, nsl - 1);
         return *(const tab_t*)(tabs + (which * TABG_MAX + kg) * CHW + chl);
     };
 
+    const v4f zero4 = v4f{0, 0, 0, 0};
+    __shared__ __attribute__((aligned(16))) float sums[DIST ? 2 * KS * 4 * MB * 16 : 4];     // [slab parity][K part][copy of lg][row]
+    const int s_wr = (ks * 4 + lg) * MB * 16 + rt * 16 + li, s_rd = (ks * 4 + lg) * MB * 16 + 4 * lg;
+    constexpr int SPAR = KS * 4 * MB * 16;
+    v4f own = zero4;             // DIST: the sums of row li of the wave's block, of a slab or (per-channel tables) of all of K
+    float nz[NH];                // DIST, group tables: -s * (8 + zp) of the slab before
+#pragma unroll
+    for (int h = 0; h < NH; ++h) nz[h] = 0.f;
     auto fold = [&](const tab_t sv, const tab_t zv) {
-        float sc[NCL], zc[NCL];
+        if constexpr (!ROWS) {
+            float sc[NCL], zc[NCL];
 #pragma unroll
-        for (int c = 0; c < NCL; ++c) {
-            const uint32_t sb = (sv[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
-            const uint32_t zb = (zv[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
-            sc[c] = bits_to_f32<SDT>(sb);
-            zc[c] = c_off + zmul * bits_to_f32<SDT>(zb);
+            for (int c = 0; c < NCL; ++c) {
+                const uint32_t sb = (sv[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
+                const uint32_t zb = (zv[c >> 1] >> (16 * (c & 1))) & 0xFFFFu;
+                sc[c] = bits_to_f32<SDT>(sb);
+                zc[c] = c_off + zmul * bits_to_f32<SDT>(zb);
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int c = NH == 2 ? 2 * r + h : r;
+                        outv[mb][h][r] += sc[c] * (accg[mb][h][r] - zc[c] * asum[mb][r]);
+                        accg[mb][h][r] = 0.f;
+                    }
+                asum[mb] = v4f{0, 0, 0, 0};
+            }
         }
+    };
+
+    // ROWS, up to 32 rows a pass: all fragments, then all MFMAs, then the fold of a group's sums
+    auto fold_rows = [&](const auto s16, const auto z16) {
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
+        for (int c = 0; c < 2; ++c) {
+            const float sc = bits_to_f32<SDT>((s16 >> (16 * c)) & 0xFFFFu), zc = -8.f - zmul * bits_to_f32<SDT>((z16 >> (16 * c)) & 0xFFFFu);
 #pragma unroll
-            for (int h = 0; h < NH; ++h)
+            for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int c = NH == 2 ? 2 * r + h : r;
-                    outv[mb][h][r] += sc[c] * (accg[mb][h][r] - zc[c] * asum[mb][r]);
-                    accg[mb][h][r] = 0.f;
+                for (int r = 0; r < 4; ++r)
+                    outv[mb][c][r] = __builtin_fmaf(sc, __builtin_fmaf(zc, asum[mb][r], accg[mb][c][r]), outv[mb][c][r]);
+        }
+    };
+    auto compute_rows = [&](const char* stage, const v4u w0, const v4u w1, const bool last, const auto& sv, const auto& zv) {
+        v4u bf[2][MB][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) bf[s][mb][h] = *(const v4u*)(stage + rd[s][h] + mb * 4096);
+        if (last) {   // partial slab: fragment (s, h) of this lane holds k = 8 * (8 s + 2 lg + h) .. + 7
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool beyond = (8 * s + 2 * lg + h) * 8 >= tail_k;
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) bf[s][mb][h] = beyond ? v4u{0, 0, 0, 0} : bf[s][mb][h];
                 }
-            asum[mb] = v4f{0, 0, 0, 0};
+        }
+        v4u w[2][2][2];         // [half of the slab][k-step][channel]
+        convert_w4_u<ADT>(w0, w[0][0][0], w[0][1][0], w[0][0][1], w[0][1][1]);
+        convert_w4_u<ADT>(w1, w[1][0][0], w[1][1][0], w[1][0][1], w[1][1][1]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool first = G128 && h == 0 && (s == 0 || GSUB == 2);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) accg[mb][c] = MT::mma(bf[s][mb][h], w[s][h][c], first ? zero4 : accg[mb][c]);
+                    asum[mb] = MT::mma(bf[s][mb][h], ones, first ? zero4 : asum[mb]);
+                }
+            if constexpr (G128 && GSUB == 2) { if (s == 0) fold_rows(sv[0], zv[0]); }
+        }
+        if constexpr (G128) fold_rows(sv[GSUB - 1], zv[GSUB - 1]);
+    };
+    // ROWS, 64 rows a pass: one block of 16 activation rows at a time - its fragments are read while the block before is multiplied,
+    // and its sums are folded while the next one is.  Both waves of a SIMD cross the same barrier, so that in the form above each of the
+    // three waits for the one before: K=8192, N=28672, groups of 128, 64 rows 52.3 -> 49.5 us; with 32 rows a pass it is the other way round,
+    // 33.8 and 36.4, with 16 they are level.
+    auto compute_rows_64 = [&](const char* stage, const v4u w0, const v4u w1, const bool last, const auto& sv, const auto& zv,
+                               float* sums_now, const float* before) {
+        v4u B[2][2][2];
+        auto read_b = [&](int mb, int at) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) B[at][s][h] = *(const v4u*)(stage + rd[s][h] + mb * 4096);
+        };
+        v4u w[2][2][2];
+        read_b(0, 0);
+        convert_w4_u<ADT>(w0, w[0][0][0], w[0][1][0], w[0][0][1], w[0][1][1]);
+        convert_w4_u<ADT>(w1, w[1][0][0], w[1][1][0], w[1][0][1], w[1][1][1]);
+        float sc[GSUB][2], zc[GSUB][2];
+        if constexpr (G128) {
+#pragma unroll
+            for (int u = 0; u < GSUB; ++u)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    sc[u][c] = bits_to_f32<SDT>((sv[u] >> (16 * c)) & 0xFFFFu);
+                    zc[u][c] = -8.f - zmul * bits_to_f32<SDT>((zv[u] >> (16 * c)) & 0xFFFFu);
+                }
+        }
+        v4f acc[2][GSUB][2], as[2][GSUB];       // group tables: a block's sums (as: of its activations, or what the waves handed on)
+#pragma unroll
+        for (int mb = 0; mb <= MB; ++mb) {
+            const int at = mb & 1, old = at ^ 1;
+            if (mb + 1 < MB) read_b(mb + 1, old);
+            else if (DIST && mb + 1 == MB) read_b(rt, old);
+            if (!G128 && last && (mb < MB || DIST)) {   // partial slab, as above
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        if ((8 * s + 2 * lg + h) * 8 >= tail_k) B[at][s][h] = v4u{0, 0, 0, 0};
+            }
+            if (mb < MB) {
+                if constexpr (DIST && G128) as[at][0] = *(const v4f*)(before + s_rd + mb * 16);
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bool first = h == 0 && (s == 0 || GSUB == 2);
+                        const int u = GSUB == 2 ? s : 0;
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            if constexpr (G128) acc[at][u][c] = MT::mma(B[at][s][h], w[s][h][c], first ? zero4 : acc[at][u][c]);
+                            else accg[mb][c] = MT::mma(B[at][s][h], w[s][h][c], accg[mb][c]);
+                        }
+                        if constexpr (!DIST && G128) as[at][u] = MT::mma(B[at][s][h], ones, first ? zero4 : as[at][u]);
+                        else if constexpr (!DIST) asum[mb] = MT::mma(B[at][s][h], ones, asum[mb]);
+                    }
+            } else if constexpr (DIST) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) own = MT::mma(ones, B[at][s][h], G128 && h == 0 && s == 0 ? zero4 : own);
+            }
+            if constexpr (G128)
+                if (mb > 0) {
+#pragma unroll
+                    for (int u = 0; u < GSUB; ++u)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const float o = outv[mb - 1][c][r], a = acc[old][u][c][r], m = as[old][u][r];
+                                outv[mb - 1][c][r] = DIST ? __builtin_fmaf(sc[u][c], a, __builtin_fmaf(nz[c], m, o))
+                                                          : __builtin_fmaf(sc[u][c], __builtin_fmaf(zc[u][c], m, a), o);
+                            }
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (DIST && G128) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) nz[c] = sc[0][c] * zc[0][c];
+            sums_now[s_wr] = own[0];
         }
     };
 
@@ -382,7 +534,19 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
         wq[W][0] = load_w((JJ) + D, 0);                                    \
         wq[W][1] = load_w((JJ) + D, 1);                                    \
         __builtin_amdgcn_sched_barrier(0);                                 \
-        if (mine_) {                                                       \
+        if constexpr (ROWS) {                                              \
+            if (mine_) {                                                   \
+                const v4u w0_ = *(const v4u*)(wmine + wrd[0]), w1_ = *(const v4u*)(wmine + wrd[1]); \
+                const bool last_ = !G128 && part_tail && (JJ) == nsl - 1;  \
+                tab_t st_[GSUB], zt_[GSUB];                                \
+                _Pragma("unroll") for (int u_ = 0; u_ < GSUB; ++u_) {      \
+                    st_[u_] = TABLDS ? lds_tab(0, (JJ)) : sq[Q][u_];       \
+                    zt_[u_] = TABLDS ? lds_tab(1, (JJ)) : zq[Q][u_];       \
+                }                                                          \
+                if constexpr (MB == 4) compute_rows_64(CUR, w0_, w1_, last_, st_, zt_, sums + ((Q) & 1) * SPAR, sums + (1 - ((Q) & 1)) * SPAR); \
+                else compute_rows(CUR, w0_, w1_, last_, st_, zt_);         \
+            }                                                              \
+        } else if (mine_) {                                                \
             bool two_step_ = false;                                        \
             if constexpr (RQBF && REFQ == 2) two_step_ = !whole_zp;        \
             if (two_step_)                                                 \
@@ -463,6 +627,7 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
         }
         __syncthreads();
     }
+    if constexpr (DIST && G128) sums[SPAR + s_wr] = 0.f;        // (read by slab 0, behind its barrier)
     static_assert(D == 4, "the unrolled loop below walks four weight slots");
     for (int jj = 0; jj < n_iter; jj += D) {
         FNN_PANEL_ITER(0, 0, st0, st3, jj);
@@ -472,8 +637,38 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
     }
 #undef FNN_PANEL_ITER
 
-    // ---- per-channel scales: one fold at the end
-    if constexpr (REFQ) {
+    // ---- DIST: what is left of the zero points (the last slab's, or all of K's); per-channel scales: one fold at the end
+    if constexpr (DIST) {
+        if constexpr (!G128) sums[s_wr] = own[0];
+        __syncthreads();
+        float sc[NH];
+        if constexpr (!G128) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                sc[h] = load_as_f32(p.scale, (MOE ? (int64_t)expert * q.stride_scale_be : 0) + n0 + h, p.scale_dtype);
+                nz[h] = -8.f - (has_zp ? load_zp_f32(p.zp, (MOE ? (int64_t)expert * q.stride_zp_be : 0) + n0 + h, p.zp_dtype) : 0.f);
+            }
+        }
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            const v4f sum = *(const v4f*)(sums + (G128 ? ((nsl - 1) & 1) * SPAR : 0) + s_rd + mb * 16);
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    outv[mb][h][r] = G128 ? __builtin_fmaf(nz[h], sum[r], outv[mb][h][r]) : sc[h] * __builtin_fmaf(nz[h], sum[r], accg[mb][h][r]);
+        }
+    } else if constexpr (ROWS && !G128) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float sc = load_as_f32(p.scale, (MOE ? (int64_t)expert * q.stride_scale_be : 0) + n0 + h, p.scale_dtype);
+            const float zc = -8.f - (has_zp ? load_zp_f32(p.zp, (MOE ? (int64_t)expert * q.stride_zp_be : 0) + n0 + h, p.zp_dtype) : 0.f);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) outv[mb][h][r] = sc * __builtin_fmaf(zc, asum[mb][r], accg[mb][h][r]);
+        }
+    } else if constexpr (REFQ) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -525,7 +720,44 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
                         outv[mb][h][r] += red[(((((k2 - 1) * RT + rt) * MB + mb) * NH + h) * 4 + r) * 64 + lane];
     }
 
-    // ---- bias, rounding, store: lane (li, lg) holds channels n0 .. n0+NCL-1 of row 16 mb + li
+    // ---- bias, rounding, store
+    if constexpr (ROWS) {       // lane (li, lg) holds channels n0, n0 + 1 of rows 16 mb + 4 lg .. + 3
+        float bias[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) bias[h] = p.bias ? load_as_f32(p.bias, n0 + h, p.bias_dtype) : 0.f;
+        const bool pairs = p.ldc % 2 == 0 && ((uintptr_t)p.out % 4) == 0;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                int m = m_base + mb * 16 + 4 * lg + r;      // output row; for gathered rows the routed-row id
+                float wroute = 1.f;
+                if constexpr (MOE) {
+                    m = token_of(mb * 16 + 4 * lg + r);
+                    if (m >= q.num_valid) continue;
+                    if (q.mul_w) wroute = load_as_f32(q.topk_w, m, q.topk_w_dtype);
+                } else {
+                    if (m >= p.M) continue;
+                }
+                uint32_t b[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    float v = outv[mb][h][r];
+                    if (p.bias) v = add_bias<WBITS>(v, bias[h], p.out_dtype);
+                    v = rounded_f32(v * wroute);
+                    b[h] = p.out_dtype == FNN_F16 ? f32_to_f16_bits(v) : f32_to_bf16_bits(v);
+                }
+                uint16_t* dst = (uint16_t*)p.out + (int64_t)m * p.ldc + n0;
+                if (pairs) {
+                    *(uint32_t*)dst = (b[0] & 0xFFFFu) | (b[1] << 16);
+                } else {
+                    dst[0] = (uint16_t)b[0];
+                    dst[1] = (uint16_t)b[1];
+                }
+            }
+        return;
+    } else {
+    // lane (li, lg) holds channels n0 .. n0+NCL-1 of row 16 mb + li
     float bias[NCL];
 #pragma unroll
     for (int c = 0; c < NCL; ++c) bias[c] = p.bias ? load_as_f32(p.bias, n0 + c, p.bias_dtype) : 0.f;
@@ -565,6 +797,7 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
 #pragma unroll
             for (int c = 0; c < NCL; ++c) dst[c] = (uint16_t)(pk[c >> 1] >> (16 * (c & 1)));
         }
+    }
     }
 }
 

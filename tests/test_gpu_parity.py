@@ -1189,6 +1189,38 @@ def test_fused_moe_a16w4_tiles_of_padding_alone_are_left_out(group):
     assert best[256] <= 1.5 * best[64], best
 
 
+@pytest.mark.parametrize("T,E,N,top_k,block,tile", [(64, 16, 4096, 2, 16, "64,128"), (400, 4, 16384, 1, 64, "128,256")])
+@pytest.mark.parametrize("K", [512, 768, 1024, 1536, 2048, 3072, 4096])
+def test_fused_moe_a16w4_tables_as_they_lie(K, T, E, N, top_k, block, tile):
+    """The tiled kernel copies its slice of the [expert, channel, group] tables as it lies: 4 to 32 groups - a row of 1, 2 or 4
+    16-byte pieces (their places are swapped), of 3, or of no whole number of them - at an address that is aligned and at one that
+    is not, which gives the same bits; sampled rows against float64."""
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    a = torch.randn(T, K, device=DEV, generator=g).bfloat16()
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    n = E * N * (K // 128)
+    tables = [torch.empty(n + 1, device=DEV).uniform_(lo, hi, generator=g).bfloat16() for lo, hi in ((1e-3, 1e-2), (-8, 8))]
+    shifted = [t[1:].view(E, N, K // 128) for t in tables]
+    aligned = [t.clone() for t in shifted]
+    assert all(t.data_ptr() % 16 == 2 for t in shifted) and all(t.data_ptr() % 16 == 0 for t in aligned)
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), top_k, dim=-1)[1].to(torch.int32)
+    w = torch.rand(T, top_k, device=DEV, generator=g)
+    s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
+
+    def run(scale, zp):
+        c = torch.empty(T, top_k, N, dtype=torch.bfloat16, device=DEV)
+        flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, True, top_k, block)
+        assert _lib.last_kernel() == f"gemm_wo_moe_kernel(group tables)<4,{tile}>", _lib.last_kernel()
+        return c.reshape(T * top_k, N)
+
+    got = run(*aligned)
+    assert torch.equal(run(*shifted), got)
+    for t in range(0, T * top_k, T * top_k // 5):
+        ex, tw = int(ids.flatten()[t]), w.flatten()[t].double()
+        want = _moe_a16w4_exact(a[t // top_k], b[ex], aligned[0][ex], aligned[1][ex]) * tw
+        assert _moe_a16w4_worst(got[t], want, a[t // top_k], aligned[0][ex], tw) <= 1.0, t
+
+
 @pytest.mark.parametrize("T,E,N,K,group,block,kernel", [
     (16, 8, 28672, 3584, 128, 16, "moe(group tables)"), (16, 8, 28672, 4096, 128, 16, "panel(moe)"),    # 28 and 32 groups
     (16, 8, 28672, 768, 0, 16, "moe"), (16, 8, 28672, 1024, 0, 16, "panel(moe)"),
