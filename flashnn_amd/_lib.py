@@ -94,6 +94,11 @@ def current_stream(device):
     return torch._C._cuda_getCurrentRawStream(idx)
 
 
+def stream_of(t):
+    """The same for the device of a tensor on a GPU (half a microsecond less: no device object is made)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
 def ptr(t):
     """Device address as an int (None -> NULL); ctypes converts it for a void* parameter."""
     return t.data_ptr() if t is not None else None

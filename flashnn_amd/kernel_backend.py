@@ -62,7 +62,7 @@ class BackendKernel(torch.nn.Module):
         return getattr(type(self), name) is not getattr(BackendKernel, name)
 
     def forward(self, *args, **kwargs):
-        if _Switches.native and self._implements("_hip_impl"):
+        if _Switches.native and type(self)._hip_impl is not BackendKernel._hip_impl:
             return self._hip_impl(*args, **kwargs)
         if self._implements("_torch_impl"):
             return self._torch_impl(*args, **kwargs)

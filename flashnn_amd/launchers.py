@@ -17,12 +17,18 @@ def hip_dynamic_quantize(out, input, scale):
     assert input.dim() == 2 and out.shape == input.shape and out.dtype == torch.int8
     assert scale.dtype == torch.float16 and scale.numel() == input.size(0)
     assert out.is_contiguous() and scale.is_contiguous()
-    _lib.require_gpu(out, input, scale)
-    lib = _lib.load()
+    return dynamic_quantize(out, input, scale)
+
+
+def dynamic_quantize(out, input, scale):
+    """hip_dynamic_quantize behind its checks."""
+    if not (out.is_cuda and input.is_cuda and scale.is_cuda):
+        _lib.require_gpu(out, input, scale)
     M, K = input.shape
-    _lib.check(lib.fnn_dynamic_quant(_lib.ptr(out), _lib.ptr(scale), _lib.ptr(input), M, K,
-                                     input.stride(0) if M > 1 else K, out.stride(0) if M > 1 else K,
-                                     _lib.dtype_code(input.dtype), _lib.current_stream(input.device)))
+    rc = _lib.load().fnn_dynamic_quant(out.data_ptr(), scale.data_ptr(), input.data_ptr(), M, K, K, K,
+                                       _lib.dtype_code(input.dtype), _lib.stream_of(input))
+    if rc:
+        _lib.check(rc)
     return out, scale
 
 
@@ -166,7 +172,8 @@ def hip_gemm_a8w8_forward(out, a, b, alpha_row, alpha_col, tile=None):
     assert out.dtype == torch.float16 or out.dtype == torch.bfloat16, \
         "Output type must be float16 or bfloat16"
     assert a.shape[1] == b.shape[1], "Matrix B must be transposed"
-    _lib.require_gpu(out, a, b, alpha_row, alpha_col)
+    if not (out.is_cuda and a.is_cuda and b.is_cuda and alpha_row.is_cuda and alpha_col.is_cuda):
+        _lib.require_gpu(out, a, b, alpha_row, alpha_col)
     lib = _lib.load()
     M, K = a.shape
     N = b.shape[0]
@@ -175,20 +182,29 @@ def hip_gemm_a8w8_forward(out, a, b, alpha_row, alpha_col, tile=None):
         b = b.contiguous()
     ar = _flat_scale(alpha_row, M, "alpha_row")
     ac = _flat_scale(alpha_col, N, "alpha_col")
-    args = (_lib.ptr(out), _lib.ptr(a), _lib.ptr(b), _lib.ptr(ar), _lib.ptr(ac),
-            M, N, K, a.stride(0) if M > 1 else K, b.stride(0) if N > 1 else K,
-            out.stride(0) if M > 1 else N, _lib.dtype_code(out.dtype),
-            _lib.dtype_code(ar.dtype), _lib.dtype_code(ac.dtype))
-    stream = _lib.current_stream(a.device)
+    code = _lib.dtype_code
+    args = (out.data_ptr(), a.data_ptr(), b.data_ptr(), ar.data_ptr(), ac.data_ptr(), M, N, K, K,
+            b.stride(0) if N > 1 else K, out.stride(0) if M > 1 else N, code(out.dtype), code(ar.dtype), code(ac.dtype))
+    stream = _lib.stream_of(a)
     # shape-keyed tuned tile, named as the reference names the launch (gemm_a8w8.py:199)
     if tile is None:
         tile = tuned_configs.CACHE.shape_tile("gemm_a8w8", M, N, K)
+    if tile is None and M <= 64 and not get_autotune_triton_kernels():
+        rc = lib.fnn_gemm_a8w8(*args, stream)
+        if rc:
+            _lib.check(rc)
+        return out
+    return _a8w8_large_or_named(lib, out, a.device, args, stream, M, N, K, tile)
+
+
+def _a8w8_large_or_named(lib, out, device, args, stream, M, N, K, tile):
+    """hip_gemm_a8w8_forward where a workspace may be needed, a tile is named or tuning is on."""
     def run_named(t):
         bm, bn, waves, parts = tuned_configs.as_config(t)
         if bm == 0:
             return run_default()
         if parts > 1:
-            ws = _a8w8_workspace_of(a.device, stream, _A8W8_WS_ALLOC)
+            ws = _a8w8_workspace_of(device, stream, _A8W8_WS_ALLOC)
             rc = lib.fnn_gemm_a8w8_ws_tiled(*args, bm, bn, parts, ws.data_ptr(), ws.numel(), stream)
             if rc != 0:
                 _A8W8_WORKSPACES.clear()
@@ -196,7 +212,7 @@ def hip_gemm_a8w8_forward(out, a, b, alpha_row, alpha_col, tile=None):
         return _lib.check(lib.fnn_gemm_a8w8_tiled(*args, bm, bn, waves, stream))
 
     def run_default():
-        ws = _a8w8_workspace(lib, a.device, stream, M, N, K) if M > 64 else None
+        ws = _a8w8_workspace(lib, device, stream, M, N, K) if M > 64 else None
         if ws is None:
             _lib.check(lib.fnn_gemm_a8w8(*args, stream))
         else:
@@ -231,12 +247,18 @@ def hip_gemm_a8w8_int32(a, b, tile=(0, 0, 0)):
     return acc
 
 
-def _weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, tile=None):
+def check_weight_only(act, quant_w):
     assert quant_w.dtype == torch.int8, "Weight must be int8 type"
     assert act.is_contiguous(), "Activation must be contiguous"
     assert quant_w.is_contiguous(), "Weight must be contiguous"
     assert act.shape[1] == quant_w.shape[1], "Matrix B must be transposed"
-    _lib.require_gpu(out, act, quant_w, scale_w, bias, zero_points)
+
+
+def weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, tile=None):
+    """The weight-only launchers behind check_weight_only."""
+    if not (out.is_cuda and act.is_cuda and quant_w.is_cuda and scale_w.is_cuda and (bias is None or bias.is_cuda) and
+            (zero_points is None or zero_points.is_cuda)):
+        _lib.require_gpu(out, act, quant_w, scale_w, bias, zero_points)
     lib = _lib.load()
     M, K = act.shape
     N = n_out
@@ -269,12 +291,35 @@ def _weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, 
         if bias.dim() != 1 or not bias.is_contiguous():
             bias = bias.reshape(-1).contiguous()
         assert bias.numel() == N
-    args = (_lib.ptr(out), _lib.ptr(act), _lib.ptr(quant_w), _lib.ptr(scale_w), _lib.ptr(bias),
-            _lib.ptr(zp), M, N, K, act.stride(0) if M > 1 else K, K,
-            out.stride(0) if M > 1 else N, group, _lib.dtype_code(act.dtype),
-            _lib.dtype_code(out.dtype), _lib.dtype_code(scale_w.dtype),
-            _lib.dtype_code(zp.dtype) if zp is not None else 0,
-            _lib.dtype_code(bias.dtype) if bias is not None else 0)
+    code = _lib.dtype_code
+    args = (out.data_ptr(), act.data_ptr(), quant_w.data_ptr(), scale_w.data_ptr(), None if bias is None else bias.data_ptr(),
+            None if zp is None else zp.data_ptr(), M, N, K, K, K, out.stride(0) if M > 1 else N, group, code(act.dtype),
+            code(out.dtype), code(scale_w.dtype), 0 if zp is None else code(zp.dtype), 0 if bias is None else code(bias.dtype))
+    stream = _lib.stream_of(act)
+    # Up to 64 rows the blocks of the few-row kernel can be named: a shape-keyed record, written by a tuning run
+    # under the name of the reference's kernel for the call (gemm_a16w8.py:84, :180; gemm_a16w4.py:84, :210) with
+    # the shape it is tuned by there (key M, N, K; gemm_a16w8.py:322-336), and the group size where there is one
+    if M <= 64:
+        prefix = _RECORD_PREFIXES.get((fn_name, group))
+        if prefix is None:
+            prefix = _RECORD_PREFIXES[fn_name, group] = fn_name[4:] + ("_per_channel" if group == 0 else f"_sub_channel_g{group}")
+        if tile is None:
+            tile = tuned_configs.CACHE.shape_tile(prefix, M, N, K)
+        if tile is None and not get_autotune_triton_kernels():
+            rc = getattr(lib, fn_name)(*args, stream)
+            if rc:
+                _lib.check(rc)
+            return out
+    else:
+        prefix = None
+    return _weight_only_large_or_named(lib, fn_name, out, act, scale_w, args, stream, M, N, K, group, tile, prefix, N // quant_w.shape[0])
+
+
+_RECORD_PREFIXES = {}       # (entry point, group size) -> what the records of its shapes are called
+
+
+def _weight_only_large_or_named(lib, fn_name, out, act, scale_w, args, stream, M, N, K, group, tile, prefix, per_byte):
+    """weight_only where scratch may be needed, blocks are named or tuning is on (prefix: where the call can be tuned)."""
     # scratch for bf16 rows converted to fp16 (so that every weight is rounded as the reference rounds it): taken
     # from torch's caching allocator per call, which hands it to later calls on this stream in stream order
     def run_default():
@@ -284,26 +329,18 @@ def _weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, 
                                                                 _lib.dtype_code(scale_w.dtype)))
         if need:
             ws = torch.empty(need, dtype=torch.uint8, device=act.device)
-            _lib.check(getattr(lib, fn_name + "_ws")(*args, ws.data_ptr(), need, _lib.current_stream(act.device)))
+            _lib.check(getattr(lib, fn_name + "_ws")(*args, ws.data_ptr(), need, stream))
         else:
-            _lib.check(getattr(lib, fn_name)(*args, _lib.current_stream(act.device)))
+            _lib.check(getattr(lib, fn_name)(*args, stream))
 
     def run_named(t):
         bm, bn = tuned_configs.as_config(t)[:2]
         if bm == 0:
             return run_default()
-        return _lib.check(getattr(lib, fn_name + "_tiled")(*args, bm, bn, _lib.current_stream(act.device)))
+        return _lib.check(getattr(lib, fn_name + "_tiled")(*args, bm, bn, stream))
 
-    # Up to 64 rows the blocks of the few-row kernel can be named: a shape-keyed record, written by a tuning run
-    # under the name of the reference's kernel for the call (gemm_a16w8.py:84, :180; gemm_a16w4.py:84, :210) with
-    # the shape it is tuned by there (key M, N, K; gemm_a16w8.py:322-336), and the group size where there is one
-    if M <= 64:
-        prefix = fn_name[4:] + ("_per_channel" if group == 0 else f"_sub_channel_g{group}")
-        if tile is None:
-            tile = tuned_configs.CACHE.shape_tile(prefix, M, N, K)
-        if tile is None and get_autotune_triton_kernels():
-            tile = tuned_configs.tune(f"{prefix}_{M}_{N}_{K}", tuned_configs.weight_only_candidates(N // quant_w.shape[0]),
-                                      run_named)
+    if tile is None and prefix is not None and get_autotune_triton_kernels():
+        tile = tuned_configs.tune(f"{prefix}_{M}_{N}_{K}", tuned_configs.weight_only_candidates(per_byte), run_named)
     if tile is None:
         run_default()
     else:
@@ -315,16 +352,18 @@ def hip_gemm_a16w8_forward(out, act, quant_w, scale_w, bias=None, zero_points=No
     """Replaces triton_gemm_a16w8_forward (flashnn/triton_kernels/gemm_a16w8.py:275-338).
     `out` need not be zeroed.  `tile` = (rows per pass, channels per workgroup) names the blocks of the few-row
     kernel (up to 64 rows) and bypasses the tuned-configuration lookup (not part of the reference's signature)."""
-    return _weight_only("fnn_gemm_a16w8", out, act, quant_w, scale_w, bias, zero_points,
-                        quant_w.shape[0], tile)
+    check_weight_only(act, quant_w)
+    return weight_only("fnn_gemm_a16w8", out, act, quant_w, scale_w, bias, zero_points,
+                       quant_w.shape[0], tile)
 
 
 def hip_gemm_a16w4_forward(out, act, quant_w, scale_w, bias=None, zero_points=None, tile=None):
     """Replaces triton_gemm_a16w4_forward (flashnn/triton_kernels/gemm_a16w4.py:336-406).
     quant_w is [N/2, K] with channel 2j in the low and 2j+1 in the high nibble of row j.  `tile` as in
     hip_gemm_a16w8_forward."""
-    return _weight_only("fnn_gemm_a16w4", out, act, quant_w, scale_w, bias, zero_points,
-                        quant_w.shape[0] * 2, tile)
+    check_weight_only(act, quant_w)
+    return weight_only("fnn_gemm_a16w4", out, act, quant_w, scale_w, bias, zero_points,
+                       quant_w.shape[0] * 2, tile)
 
 
 class PrepackedInt4:

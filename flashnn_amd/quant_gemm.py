@@ -8,14 +8,15 @@ import torch
 
 from . import torch_formulas
 from .kernel_backend import BackendKernel
-from .launchers import (hip_a16w4_prepack, hip_dynamic_quantize, hip_gemm_a8w8_forward, hip_gemm_a16w4_forward,
-                        hip_gemm_a16w4_prepacked_forward, hip_gemm_a16w8_forward)
+from .launchers import (check_weight_only, dynamic_quantize, hip_a16w4_prepack, hip_gemm_a8w8_forward,
+                        hip_gemm_a16w4_prepacked_forward, weight_only)
 
 
 def _weight_type(quant_w, scale_w):
-    if quant_w.size(0) == scale_w.size(-1) / 2:
+    rows, channels = quant_w.size(0), scale_w.size(-1)
+    if rows * 2 == channels:
         return torch.quint4x2
-    if quant_w.size(0) == scale_w.size(-1):
+    if rows == channels:
         return torch.int8
     return None
 
@@ -34,8 +35,9 @@ class DynamicQuantize(BackendKernel):
     def _hip_impl(self, input):
         out = torch.empty(input.shape, dtype=torch.int8, device=input.device)
         scale = torch.empty(input.shape[0], dtype=torch.half, device=input.device)
-        hip_dynamic_quantize(out, input, scale)
-        return out, scale
+        assert input.is_contiguous(), "input must be contiguous"
+        assert input.dim() == 2
+        return dynamic_quantize(out, input, scale)
 
     def forward(self, input):
         return BackendKernel.forward(self, input)
@@ -69,21 +71,16 @@ class GemmWeightOnly(BackendKernel):
         self.out_ty = out_ty
 
     def _hip_impl(self, act, quant_w, scale_w, bias=None, zero_points=None):
-        assert quant_w.dtype == torch.int8, "Weight must be int8 type"
-        assert act.is_contiguous(), "Activation must be contiguous"
-        assert quant_w.is_contiguous(), "Weight must be contiguous"
-        assert act.shape[1] == quant_w.shape[1], "Matrix B must be transposed"
+        check_weight_only(act, quant_w)
         weight_type = _weight_type(quant_w, scale_w)
         if weight_type == torch.int8:
-            out = torch.empty([act.shape[0], quant_w.shape[0]], dtype=self.out_ty, device=act.device)
-            hip_gemm_a16w8_forward(out, act, quant_w, scale_w, bias=bias, zero_points=zero_points)
+            entry, channels = "fnn_gemm_a16w8", quant_w.shape[0]
         elif weight_type == torch.quint4x2:
-            out = torch.empty([act.shape[0], quant_w.shape[0] * 2], dtype=self.out_ty,
-                              device=act.device)
-            hip_gemm_a16w4_forward(out, act, quant_w, scale_w, bias=bias, zero_points=zero_points)
+            entry, channels = "fnn_gemm_a16w4", quant_w.shape[0] * 2
         else:
             raise AssertionError("Gemm WeightOnly only support int8 or int4x2")
-        return out
+        out = torch.empty((act.shape[0], channels), dtype=self.out_ty, device=act.device)
+        return weight_only(entry, out, act, quant_w, scale_w, bias, zero_points, channels)
 
     def _torch_impl(self, act, quant_w, scale_w, bias=None, zero_points=None):
         assert act.shape[1] == quant_w.shape[1], "Matrix B must be transposed"
