@@ -31,7 +31,7 @@
 
 namespace fnn {
 
-// K / 128 at most, where there are group tables: they lie in LDS whole, 33 KB for 32 groups of 256 channels beside 112 KB of
+// K / 128 at most, where there are group tables: they lie in LDS whole, 32 KB for 32 groups of 256 channels beside 112 KB of
 // stages, and 64 groups do not fit the 160 KB.  Longer rows (K = 4224 to 8192) stay on gemm_wo_tile_kernel and the panel kernel.
 constexpr int kGroups = 32;
 
