@@ -13,15 +13,21 @@ from .kernel_backend import get_autotune_triton_kernels
 
 def hip_dynamic_quantize(out, input, scale):
     """Replaces triton_dynamic_quantize (flashnn/triton_kernels/dynamic_quant.py:73-97)."""
-    assert input.is_contiguous(), "input must be contiguous"
-    assert input.dim() == 2 and out.shape == input.shape and out.dtype == torch.int8
+    _check_dynamic_quantize(input)
+    assert out.shape == input.shape and out.dtype == torch.int8
     assert scale.dtype == torch.float16 and scale.numel() == input.size(0)
     assert out.is_contiguous() and scale.is_contiguous()
-    return dynamic_quantize(out, input, scale)
+    return _dynamic_quantize(out, input, scale)
 
 
-def dynamic_quantize(out, input, scale):
-    """hip_dynamic_quantize behind its checks."""
+def _check_dynamic_quantize(input):
+    """What callers of _dynamic_quantize check of an input; outputs that they allocate by it need no checks."""
+    assert input.is_contiguous(), "input must be contiguous"
+    assert input.dim() == 2
+
+
+def _dynamic_quantize(out, input, scale):
+    """hip_dynamic_quantize behind its checks: contiguous matrices, whose rows are K apart."""
     if not (out.is_cuda and input.is_cuda and scale.is_cuda):
         _lib.require_gpu(out, input, scale)
     M, K = input.shape
@@ -247,15 +253,16 @@ def hip_gemm_a8w8_int32(a, b, tile=(0, 0, 0)):
     return acc
 
 
-def check_weight_only(act, quant_w):
+def _check_weight_only(act, quant_w):
+    """What callers of _weight_only check before they work out the number of channels."""
     assert quant_w.dtype == torch.int8, "Weight must be int8 type"
     assert act.is_contiguous(), "Activation must be contiguous"
     assert quant_w.is_contiguous(), "Weight must be contiguous"
     assert act.shape[1] == quant_w.shape[1], "Matrix B must be transposed"
 
 
-def weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, tile=None):
-    """The weight-only launchers behind check_weight_only."""
+def _weight_only(fn_name, out, act, quant_w, scale_w, bias, zero_points, n_out, tile=None):
+    """The weight-only launchers behind _check_weight_only: contiguous activations and weights, whose rows are K apart."""
     if not (out.is_cuda and act.is_cuda and quant_w.is_cuda and scale_w.is_cuda and (bias is None or bias.is_cuda) and
             (zero_points is None or zero_points.is_cuda)):
         _lib.require_gpu(out, act, quant_w, scale_w, bias, zero_points)
@@ -319,7 +326,7 @@ _RECORD_PREFIXES = {}       # (entry point, group size) -> what the records of i
 
 
 def _weight_only_large_or_named(lib, fn_name, out, act, scale_w, args, stream, M, N, K, group, tile, prefix, per_byte):
-    """weight_only where scratch may be needed, blocks are named or tuning is on (prefix: where the call can be tuned)."""
+    """_weight_only where scratch may be needed, blocks are named or tuning is on (prefix: where the call can be tuned)."""
     # scratch for bf16 rows converted to fp16 (so that every weight is rounded as the reference rounds it): taken
     # from torch's caching allocator per call, which hands it to later calls on this stream in stream order
     def run_default():
@@ -352,18 +359,18 @@ def hip_gemm_a16w8_forward(out, act, quant_w, scale_w, bias=None, zero_points=No
     """Replaces triton_gemm_a16w8_forward (flashnn/triton_kernels/gemm_a16w8.py:275-338).
     `out` need not be zeroed.  `tile` = (rows per pass, channels per workgroup) names the blocks of the few-row
     kernel (up to 64 rows) and bypasses the tuned-configuration lookup (not part of the reference's signature)."""
-    check_weight_only(act, quant_w)
-    return weight_only("fnn_gemm_a16w8", out, act, quant_w, scale_w, bias, zero_points,
-                       quant_w.shape[0], tile)
+    _check_weight_only(act, quant_w)
+    return _weight_only("fnn_gemm_a16w8", out, act, quant_w, scale_w, bias, zero_points,
+                        quant_w.shape[0], tile)
 
 
 def hip_gemm_a16w4_forward(out, act, quant_w, scale_w, bias=None, zero_points=None, tile=None):
     """Replaces triton_gemm_a16w4_forward (flashnn/triton_kernels/gemm_a16w4.py:336-406).
     quant_w is [N/2, K] with channel 2j in the low and 2j+1 in the high nibble of row j.  `tile` as in
     hip_gemm_a16w8_forward."""
-    check_weight_only(act, quant_w)
-    return weight_only("fnn_gemm_a16w4", out, act, quant_w, scale_w, bias, zero_points,
-                       quant_w.shape[0] * 2, tile)
+    _check_weight_only(act, quant_w)
+    return _weight_only("fnn_gemm_a16w4", out, act, quant_w, scale_w, bias, zero_points,
+                        quant_w.shape[0] * 2, tile)
 
 
 class PrepackedInt4:

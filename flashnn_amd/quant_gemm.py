@@ -8,8 +8,8 @@ import torch
 
 from . import torch_formulas
 from .kernel_backend import BackendKernel
-from .launchers import (check_weight_only, dynamic_quantize, hip_a16w4_prepack, hip_gemm_a8w8_forward,
-                        hip_gemm_a16w4_prepacked_forward, weight_only)
+from .launchers import (_check_dynamic_quantize, _check_weight_only, _dynamic_quantize, _weight_only, hip_a16w4_prepack,
+                        hip_gemm_a8w8_forward, hip_gemm_a16w4_prepacked_forward)
 
 
 def _weight_type(quant_w, scale_w):
@@ -35,9 +35,8 @@ class DynamicQuantize(BackendKernel):
     def _hip_impl(self, input):
         out = torch.empty(input.shape, dtype=torch.int8, device=input.device)
         scale = torch.empty(input.shape[0], dtype=torch.half, device=input.device)
-        assert input.is_contiguous(), "input must be contiguous"
-        assert input.dim() == 2
-        return dynamic_quantize(out, input, scale)
+        _check_dynamic_quantize(input)
+        return _dynamic_quantize(out, input, scale)
 
     def forward(self, input):
         return BackendKernel.forward(self, input)
@@ -71,7 +70,7 @@ class GemmWeightOnly(BackendKernel):
         self.out_ty = out_ty
 
     def _hip_impl(self, act, quant_w, scale_w, bias=None, zero_points=None):
-        check_weight_only(act, quant_w)
+        _check_weight_only(act, quant_w)
         weight_type = _weight_type(quant_w, scale_w)
         if weight_type == torch.int8:
             entry, channels = "fnn_gemm_a16w8", quant_w.shape[0]
@@ -80,7 +79,7 @@ class GemmWeightOnly(BackendKernel):
         else:
             raise AssertionError("Gemm WeightOnly only support int8 or int4x2")
         out = torch.empty((act.shape[0], channels), dtype=self.out_ty, device=act.device)
-        return weight_only(entry, out, act, quant_w, scale_w, bias, zero_points, channels)
+        return _weight_only(entry, out, act, quant_w, scale_w, bias, zero_points, channels)
 
     def _torch_impl(self, act, quant_w, scale_w, bias=None, zero_points=None):
         assert act.shape[1] == quant_w.shape[1], "Matrix B must be transposed"

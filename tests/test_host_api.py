@@ -162,6 +162,33 @@ def test_launcher_asserts_match_the_reference_messages():
                                torch.empty(4).half())
 
 
+def test_launchers_without_checks_are_private_and_callers_share_the_checks():
+    """Every public function of the launchers module checks what it is handed; the operators, which call the bodies behind
+    the checks, refuse what the launchers refuse, with the same message."""
+    import inspect
+
+    from flashnn_amd import launchers as L
+    public = [n for n, f in inspect.getmembers(L, inspect.isfunction) if f.__module__ == L.__name__ and not n.startswith("_")]
+    assert public and all(n.startswith("hip_") for n in public), public
+
+    def message(call):
+        with pytest.raises(AssertionError) as err:
+            call()
+        return str(err.value).split("\n")[0]
+
+    q, s = torch.empty(4, 64, dtype=torch.int8), torch.empty(4).half()
+    for x in (torch.zeros(4, 128).half()[:, ::2], torch.zeros(64, 4).half().t(), torch.zeros(8, 64).half()[::2],
+              torch.zeros(2, 2, 64).half(), torch.zeros(64).half()):
+        assert message(lambda: flashnn_amd.DynamicQuantize()(x)) == message(lambda: L.hip_dynamic_quantize(q, x, s))
+    act, w, sc, out = torch.zeros(4, 64).half(), torch.zeros(8, 64, dtype=torch.int8), torch.ones(8).half(), torch.empty(4, 8).half()
+    for bad_act, bad_w in ((act, w.float()), (torch.zeros(4, 128).half()[:, ::2], w), (act, w.t().contiguous().t()),
+                           (act, torch.zeros(16, 64, dtype=torch.int8)[::2]), (torch.zeros(4, 32).half(), w)):
+        for bits, fwd in ((8, L.hip_gemm_a16w8_forward), (4, L.hip_gemm_a16w4_forward)):
+            scale = sc if bits == 8 else torch.ones(16).half()
+            assert message(lambda: flashnn_amd.GemmWeightOnly()(bad_act, bad_w, scale)) == \
+                message(lambda: fwd(out, bad_act, bad_w, scale))
+
+
 def test_tuned_config_file_format_and_lookup(tmp_path, monkeypatch):
     """The tuned-configuration cache keeps the reference's file format
     (flashnn/triton_kernels/triton_utils.py:38-57, 60-75): {method_name: [kwargs, launch options]}."""
