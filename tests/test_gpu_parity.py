@@ -1041,16 +1041,34 @@ def _moe_a16w4_exact(a, packed, scale, zp):
 
 def _moe_a16w4_worst(got, want, a, scale, weight):
     """The largest of a row's errors over what is allowed, 1 and less being in order.  Value by value: one rounding to 16 bits and
-    the fp32 sums of 128 products a * (c + q), c = 1032 or 136, each at most 128 2^-24 of their magnitudes before c and the zero
-    point come off.  That is a worst case and several per cent of a small result, so the row as a whole must also lie
-    within 1e-3 (bf16: 5e-3) of its 2-norm, about five (three) times what the output's rounding alone gives."""
+    the fp32 sums of 128 products of a group (or of all of K, per-channel tables), each at most 128 2^-24 of their magnitudes:
+    a * u with u = q + 8 up to 15, and what comes off, 8 + zp times a, with zp from -8 to 8 up to 16.  That is a worst case and
+    more than a small result, so the row as a whole must also lie within 2^-11 (bf16: 2^-8) of its 2-norm, the most that the
+    output's rounding alone can give and about twice what it does give."""
     fp16 = got.dtype == torch.float16
     K, N = a.shape[0], scale.shape[0]
-    slabs = a.double().abs().reshape(K // 128, 128).sum(1) * (1048.0 if fp16 else 152.0)
-    mags = (slabs * scale.double().reshape(N, -1)).sum(1)          # (per-channel tables: one scale for all slabs)
-    bound = want.abs() * (2.0 ** -11 if fp16 else 2.0 ** -8) * 1.01 + mags * 2.0 ** -24 * 128 * weight + 1e-7
+    G = 1 if scale.dim() == 1 else scale.shape[1]
+    mags = ((a.double().abs().reshape(G, K // G).sum(1) * (15.0 + 16.0)) * scale.double().reshape(N, G)).sum(1)
+    rounding = 2.0 ** -11 if fp16 else 2.0 ** -8
+    bound = want.abs() * rounding * 1.01 + mags * 2.0 ** -24 * 128 * weight + 1e-7
     err = (got.double() - want).abs()
-    return max(float((err / bound).max()), float(err.norm() / want.norm()) / (1e-3 if fp16 else 5e-3))
+    return max(float((err / bound).max()), float(err.norm() / want.norm()) / rounding)
+
+
+def _moe_a16w4_flips(got, want, a, scale, slabs):
+    """Values of a row that are not the correctly rounded result, and how many may be, where the activations' share comes off every
+    `slabs` slabs of 128 (for activations of one sign and zero points of a channel that are the same in all its groups: the sums
+    grow towards the result).  A value's error in fp32 moves it over a rounding boundary with a chance of that error over the
+    distance between two 16-bit numbers, so the count shows errors a thousandth of the output's rounding.  The error:
+    an fp32 sum of at most R = the result and 8 times the activations of `slabs` slabs, rounded by K / 32 MFMAs of the products and as
+    many of the activations, each taken as two roundings (what an MFMA rounds inside), uniform in half a last place and independent:
+    2^-24 R sqrt(4 K / 32 / 3), of which the mean magnitude is 0.8."""
+    digits = 10 if got.dtype == torch.float16 else 7
+    step = 2.0 ** (torch.floor(torch.log2(want.abs())) - digits)
+    scale = scale.double().reshape(want.numel(), -1).mean(1)
+    most = want.abs() + scale * 8 * 128 * slabs * float(a.double().abs().mean())
+    sigma = 2.0 ** -24 * most * (4 * a.shape[0] / 32 / 3) ** 0.5
+    return int((got != want.to(got.dtype)).sum()), float((0.8 * sigma / step).sum())
 
 
 @pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
@@ -1104,34 +1122,34 @@ def test_fused_moe_a16w4_blocks_put_together(shape, group, with_zp, act_ty):
     assert torch.equal(part[listed], got.reshape(M * top_k, N)[listed]) and bool((part[~listed] == 3.0).all())
 
 
-@pytest.mark.parametrize("K,block", [(14336, 16), (14336, 64), (14336, 256), (1024, 16)])
-def test_fused_moe_a16w4_per_channel_error_does_not_grow_with_k(K, block):
-    """Per-channel tables and activations that do not cancel (all positive, as behind a ReLU): what the tiled kernel adds to
-    the rounding of the output (fp16: bf16's hides it).  The nibbles ride on an offset c, so a slab of 128 carries sums of 128
-    c mean|a|; each of its roundings (taken as eight: four MFMAs, the fold, and what an MFMA rounds inside; twice the whole is
-    allowed) is at most 2^-24 of them, and the slabs' errors add up as independent ones do."""
+@pytest.mark.parametrize("K,block,group", [(14336, 16, 0), (14336, 64, 0), (14336, 256, 0), (1024, 16, 0), (4096, 64, 128), (2048, 16, 128)])
+def test_fused_moe_a16w4_error_does_not_grow_with_k(K, block, group):
+    """Activations that do not cancel (all positive, as behind a ReLU), weights that nearly do (zero points of -1 and 0): the sums
+    that the tiled kernel carries are those of eight slabs (per-channel tables) or one and not of all of K, and the nibbles' offset
+    is 8, which shows in how many values are not the correctly rounded ones (_moe_a16w4_flips, three standard deviations of
+    the count on top)."""
     T, E, N, top_k, act_ty = 200, 4, 4096, 2, torch.float16
     g = torch.Generator(device=DEV).manual_seed(K + block)
     a = torch.randn(T, K, device=DEV, generator=g).abs().to(act_ty)
     b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
-    scale = torch.empty(E, N, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
-    zp = torch.randint(-8, 8, (E, N), device=DEV, generator=g).to(act_ty)
+    tables = (E, N, K // 128) if group else (E, N)
+    scale = torch.empty(tables, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
+    zp = torch.randint(-1, 1, (E, N, 1) if group else (E, N), device=DEV, generator=g).to(act_ty).expand(tables).contiguous()
     ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), top_k, dim=-1)[1].to(torch.int32)
     w = torch.ones(T, top_k, device=DEV)
     s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), block, E)]
     c = torch.empty(T, top_k, N, dtype=act_ty, device=DEV)
     flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, False, top_k, block)
-    assert _lib.last_kernel().startswith("gemm_wo_moe_kernel<4,"), _lib.last_kernel()
-    rows = range(0, T * top_k, 25)
-    want = torch.stack([_moe_a16w4_exact(a[t // top_k], b[ex], scale[ex], zp[ex])
-                        for t in rows for ex in [int(ids.flatten()[t])]])
-    norm = float(want.norm())
-    err = float((c.reshape(T * top_k, N)[list(rows)].double() - want).norm()) / norm
-    rounding = float((want.to(act_ty).double() - want).norm()) / norm
-    slab = 128 * 1048.0 * float(a.double().mean())
-    added = 2 * 2.0 ** -24 * slab * (8 * K / 128) ** 0.5 * float(scale.double().square().mean().sqrt()) / float(
-        want.square().mean().sqrt())
-    assert err ** 2 <= rounding ** 2 * (1 + 1e-3) + added ** 2, (err, rounding, added)
+    assert _lib.last_kernel().startswith(f"gemm_wo_moe_kernel{'(group tables)' if group else ''}<4,"), _lib.last_kernel()
+    flips = allowed = 0
+    for t in range(0, T * top_k, 25):
+        ex = int(ids.flatten()[t])
+        want = _moe_a16w4_exact(a[t // top_k], b[ex], scale[ex], zp[ex])
+        got = c.reshape(T * top_k, N)[t]
+        assert _moe_a16w4_worst(got, want, a[t // top_k], scale[ex], 1.0) <= 1.0, t
+        n, most = _moe_a16w4_flips(got, want, a[t // top_k], scale[ex], 1 if group else 8)
+        flips, allowed = flips + n, allowed + most
+    assert flips <= allowed + 3 * allowed ** 0.5, (flips, allowed)
 
 
 @pytest.mark.parametrize("T,N,block,tile", [

@@ -628,3 +628,46 @@ def test_moe_a16w4_row_check_finds_planted_mistakes(K, group, act_ty):
     assert worst(_moe_a16w4_exact(without, packed, scale, zp)) > 1.0
     other = ((packed << 4) & -16) | ((packed >> 4) & 15)
     assert worst(_moe_a16w4_exact(a, other, scale, zp)) > 1.0
+
+
+def _moe_a16w4_fp32_model(a, packed, scale, zp, slabs, c=8):
+    """A row of the tiled A16W4 kernel's arithmetic: sums of a * (q + c) in fp32, one rounding per 32 products, the sums of a beside
+    them.  Per-channel tables: (c + zp) times those taken off every `slabs` slabs of 128; groups of 128: scaled and added up
+    slab by slab."""
+    K, N = a.shape[0], scale.shape[0]
+    fp32 = lambda x: x.float().double()
+    u = torch.stack([(packed << 4) >> 4, packed >> 4], 1).reshape(N, K).double() + c
+    products, sums = (u * a.double()).reshape(N, K // 32, 32).sum(2), a.double().reshape(K // 32, 32).sum(1)
+    out, acc, own = (torch.zeros(n, dtype=torch.float64) for n in (N, N, 1))
+    for i in range(K // 32):
+        acc, own = fp32(acc + products[:, i]), fp32(own + sums[i])
+        if scale.dim() == 2 and i % 4 == 3:
+            sc = scale[:, i // 4].double()
+            out = fp32(fp32(out - fp32(sc * (c + zp[:, i // 4].double())) * own) + sc * acc)
+            acc, own = acc * 0, own * 0
+        elif scale.dim() == 1 and ((i + 1) % (4 * slabs) == 0 or i + 1 == K // 32):
+            acc, own = fp32(acc - (c + zp.double()) * own), own * 0
+    return (out if scale.dim() == 2 else fp32(acc * scale.double())).to(a.dtype)
+
+
+@pytest.mark.parametrize("K,group", [(14336, 0), (4096, 128)])
+def test_moe_a16w4_flips_find_sums_that_are_too_large(K, group):
+    """What the GPU tests hold the kernel to: a model of its arithmetic passes; one that takes the activations' share of
+    per-channel tables off once, at the end of K, or that carries q + 1032 through the groups, does not."""
+    from test_gpu_parity import _moe_a16w4_exact, _moe_a16w4_flips
+    N, slabs = 2048, 1 if group else 8
+    g = torch.Generator().manual_seed(3)
+    models = {"kernel": (slabs, 8), "planted": (1, 1032) if group else (K // 128, 8)}
+    count = dict.fromkeys(models, 0)
+    allowed = 0.0
+    for _ in range(8):
+        a = torch.randn(K, generator=g).abs().half()
+        packed = torch.randint(-128, 128, (N // 2, K), dtype=torch.int8, generator=g)
+        scale = torch.empty((N, K // 128) if group else (N,)).uniform_(1e-3, 1e-2, generator=g).half()
+        zp = torch.randint(-1, 1, (N, 1) if group else (N,), generator=g).half().expand(scale.shape)
+        want = _moe_a16w4_exact(a, packed, scale, zp)
+        for name, form in models.items():
+            flips, most = _moe_a16w4_flips(_moe_a16w4_fp32_model(a, packed, scale, zp, *form), want, a, scale, slabs)
+            count[name] += flips
+        allowed += most
+    assert count["kernel"] <= allowed + 3 * allowed ** 0.5 < count["planted"], (count, allowed)
