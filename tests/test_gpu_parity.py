@@ -1717,6 +1717,75 @@ def test_weight_only_tiled_zero_points_whole_or_not(bits, group, kind, ty):
     assert _lib.last_kernel().startswith("gemm_wo_tile_kernel(per-weight rounding)"), _lib.last_kernel()
 
 
+def _wo_int4_rows(got, act, qw, scale, zp):
+    """Every row against float64 products (_moe_a16w4_worst: u = q + 8, scaled in fp32, one rounding of the output)."""
+    sc = scale if scale.dim() == 1 else scale.t().contiguous()
+    z = None if zp is None else zp if zp.dim() == 1 else zp.t().contiguous()
+    for m in range(got.shape[0]):
+        want = _moe_a16w4_exact(act[m], qw, sc, z)
+        worst = _moe_a16w4_worst(got[m], want, act[m], sc, 1.0)
+        assert worst <= 1.0, (m, worst)
+
+
+@pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("with_zp", [True, False])
+@pytest.mark.parametrize("K,group", [(1152, 128), (1280, 128), (2176, 128), (1056, 0), (1088, 0), (1152, 0), (8896, 0), (1024, 64), (1152, 64)])
+def test_weight_only_int4_64_rows_a_pass(K, group, with_zp, act_ty):
+    """The few-row kernel's build for 64 rows a pass over int4 weights scaled in fp32, with its blocks named: parts of K of 4 and 5, 5
+    and 5, 8 and 9 slabs (the activation sums that are handed on end in one buffer or the other), a last slab of 32, 64 and none of 128
+    values missing, groups of 64 (no sums handed on); 33 and 64 rows in one pass."""
+    N = 1280
+    g = torch.Generator(device=DEV).manual_seed(K + group)
+    table_ty = torch.bfloat16 if act_ty == torch.float16 else torch.float16     # (one type for both: rounded per weight, without groups)
+    act = torch.randn(64, K, device=DEV, generator=g).to(act_ty)
+    qw = torch.randint(-128, 128, (N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    tables = (K // group, N) if group else (N,)
+    scale = torch.empty(tables, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(table_ty)
+    zp = torch.randint(-8, 8, tables, device=DEV, generator=g).to(table_ty) if with_zp else None
+    for M in (33, 64):
+        out = torch.full((M, N), float("nan"), dtype=act_ty, device=DEV)
+        launchers.hip_gemm_a16w4_forward(out, act[:M], qw, scale, None, zp, tile=(64, 128))
+        assert _lib.last_kernel() == "gemm_wo_panel_kernel<4,4,4>", _lib.last_kernel()
+        _wo_int4_rows(out, act, qw, scale, zp)
+
+
+@pytest.mark.parametrize("M,N,K,group", [(100, 16384, 1152, 128), (40, 28672, 1152, 128), (40, 28672, 1056, 0)])
+def test_weight_only_int4_64_rows_a_pass_by_the_librarys_choice(M, N, K, group):
+    """The same build where the library takes it by itself: two passes, and wide matrices."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    act = torch.randn(M, K, device=DEV, generator=g).half()
+    qw = torch.randint(-128, 128, (N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    tables = (K // group, N) if group else (N,)
+    scale = torch.empty(tables, device=DEV).uniform_(1e-3, 1e-2, generator=g).bfloat16()
+    zp = torch.randint(-8, 8, tables, device=DEV, generator=g).bfloat16()
+    out = flashnn_amd.GemmWeightOnly(torch.float16)(act, qw, scale, None, zp)
+    assert _lib.last_kernel() == "gemm_wo_panel_kernel<4,4,4>", _lib.last_kernel()
+    _wo_int4_rows(out, act, qw, scale, zp)
+
+
+@pytest.mark.parametrize("act_ty", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [1056, 1152, 1376])
+def test_fused_moe_a16w4_64_rows_a_pass(K, act_ty):
+    """The gathered form of that build: per-channel tables in blocks of 64, rows that the tiled kernel does not take (K no multiple
+    of 256), a partial last slab and parts of 4 and 5 slabs."""
+    T, E, N = 60, 3, 28672
+    g = torch.Generator(device=DEV).manual_seed(K)
+    a = torch.randn(T, K, device=DEV, generator=g).to(act_ty)
+    b = torch.randint(-128, 128, (E, N // 2, K), dtype=torch.int8, device=DEV, generator=g)
+    scale = torch.empty(E, N, device=DEV).uniform_(1e-3, 1e-2, generator=g).to(act_ty)
+    zp = torch.randint(-8, 8, (E, N), device=DEV, generator=g).to(act_ty)
+    ids = torch.topk(torch.rand(T, E, device=DEV, generator=g), 2, dim=-1)[1].to(torch.int32)
+    w = torch.rand(T, 2, device=DEV, generator=g)
+    s, e, used = [t.to(DEV) for t in workloads.moe_align_block_size(ids.cpu(), 64, E)]
+    c = torch.empty(T, 2, N, dtype=act_ty, device=DEV)
+    flashnn_amd.fused_moe_a16w4_forward(a, b, c, scale, zp, w, ids, s, e, used, True, 2, 64)
+    assert _lib.last_kernel() == "gemm_wo_panel_kernel(moe)<4,4,4>", _lib.last_kernel()
+    for t in range(0, 2 * T, 7):
+        ex, tw = int(ids.flatten()[t]), w.flatten()[t].double()
+        want = _moe_a16w4_exact(a[t // 2], b[ex], scale[ex], zp[ex]) * tw
+        assert _moe_a16w4_worst(c.reshape(2 * T, N)[t], want, a[t // 2], scale[ex], tw) <= 1.0, t
+
+
 def _close_to(got, want, out_ty):
     """Two fp32 summation orders of one dot product, each rounded once to the output type."""
     got, want = got.float().cpu().numpy(), want.float().cpu().numpy()

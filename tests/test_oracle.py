@@ -671,3 +671,23 @@ def test_moe_a16w4_flips_find_sums_that_are_too_large(K, group):
             count[name] += flips
         allowed += most
     assert count["kernel"] <= allowed + 3 * allowed ** 0.5 < count["planted"], (count, allowed)
+
+
+@pytest.mark.parametrize("K,group", [(1152, 128), (1056, 0)])
+def test_int4_row_check_finds_sums_of_another_slab_and_a_tail_that_is_counted(K, group):
+    """Mistakes that the few-row kernel could make with sums handed on a slab later: the last slab's zero points taken off with the
+    sums of the slab before, and values beyond a partial last slab (here: its first 32 once more) among the sums."""
+    from test_gpu_parity import _moe_a16w4_exact, _moe_a16w4_worst
+    N = 256
+    g = torch.Generator().manual_seed(K)
+    a = torch.randn(K, generator=g).half()
+    packed = torch.randint(-128, 128, (N // 2, K), dtype=torch.int8, generator=g)
+    scale = torch.empty((N, K // 128) if group else (N,)).uniform_(1e-3, 1e-2, generator=g).half()
+    zp = torch.randint(-8, 8, scale.shape, generator=g).half()
+    want = _moe_a16w4_exact(a, packed, scale, zp)
+    last = (lambda t: t[:, -1].double()) if group else (lambda t: t.double())
+    sums = a.double()[:K // 128 * 128].reshape(-1, 128).sum(1)
+    off = sums[-1] - sums[-2] if group else a.double()[-32:].sum()
+    worst = lambda row: _moe_a16w4_worst(row.half(), want, a, scale, 1.0)
+    assert worst(want) <= 1.0
+    assert worst(want + last(scale) * (8 + last(zp)) * off) > 1.0
