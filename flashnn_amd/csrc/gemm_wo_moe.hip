@@ -15,15 +15,19 @@
 // up one fragment and hands the sums on through LDS; they are used a slab later, so that no barrier is added.  Tables are copied into LDS
 // as they lie, once per tile.  A tile whose upper half holds padding alone (the last one of an expert) does half the work.
 //
-// What bounds it: a slab of the 128 x 256 tile has 68 MFMAs, 208 other vector instructions (fold 128, conversion 56) and 43 LDS reads per
-// wave.  In a loop of the same instructions on LDS contents, without copies, an MFMA takes 12.3 ns (two waves a SIMD; 7.9 alone, 8.7
-// with the first half of the fold, 10.8 with the whole fold and the conversion, the rest is the fragments' way from LDS); the kernel takes 13.2.
+// What bounds it: a slab of the 128 x 256 tile has per wave 68 MFMAs, 217 other vector instructions (fold 128, conversion 56) and 50 LDS
+// reads (36 of fragments, 8 of sums, 2 of weights, 4 table entries), of which none alone fills the 1.8 us that it takes: the MFMAs of a
+// SIMD's two waves take 1.07 us by themselves, the CU's 304 KB of fragments and weights 0.63 (LDS reads of this pattern run at 480
+// bytes/ns, eight waves and nothing else).  In a loop of such instructions on LDS contents, without copies, an MFMA takes 12.3 ns (two
+// waves a SIMD; 7.9 alone, 8.7 with the first half of the fold, 10.8 with the whole fold and the conversion, the rest is the fragments'
+// way from LDS); the kernel takes 13.2.
 // About 20 of a tile's 136 thousand cycles are spent before the first slab and behind the last.  Wave tiles of 64 x 64 read half the fragments
 // and convert twice the weights: the same within 2 %; the waves of a SIMD half a slab apart, the conversion a slab ahead, fragments read two
 // ahead, copies at the slab's start or spread over it: no difference.
-// 8 experts of N=28672 K=4096, groups of 128, bf16, 1024 tokens in blocks of 64, us: 745 -> 570 (830 TFLOP/s; 128 rows x 64 channels of
-// every wave in two rows of waves, sums of the activations in every wave, 136 or 1032 + q as operands, tables transposed by 2-byte stores:
-// 745); over 716 calls of 11 layers 5 to 30 % less than that form wherever this kernel has them.
+// 8 experts of N=28672 K=4096, groups of 128, bf16, 1024 tokens in blocks of 64, us of a call among others: 741 -> 594 (810 TFLOP/s) on one
+// box, 736 -> 580 on another (before: 128 rows x 64 channels of every wave in two rows of waves, sums of the activations in every wave, 136
+// or 1032 + q as operands, tables transposed by 2-byte stores); over 716 calls of 11 layers 5 to 30 % less than that form wherever
+// this kernel has them.
 #include <cmath>
 #include <type_traits>
 
@@ -52,7 +56,7 @@ __device__ __forceinline__ void moe_tile(const WoArgs& p, const MoeArgs& q, cons
     __shared__ __attribute__((aligned(1024))) char tab_s[GROUPS ? kGroups * BN * 2 : 1024], tab_z[GROUPS ? kGroups * BN * 2 : 1024];
     __shared__ __attribute__((aligned(16))) int toks[BM];
     __shared__ __attribute__((aligned(16))) float factors[BM];                       // routing weights
-    __shared__ __attribute__((aligned(16))) float sums[(GROUPS ? 2 : 1) * 4 * BM];   // activation sums of a slab's rows (of all of K), four copies
+    __shared__ __attribute__((aligned(16))) float sums[(GROUPS ? 2 : 1) * 4 * BM];   // activation sums of a slab's rows (per-channel tables: of eight slabs), four copies
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -391,9 +395,13 @@ bool launch_wo_moe_tiled(WoArgs& p, const MoeArgs& q, int act_dtype, hipStream_t
     // 4 experts N=16384 K=5120: 64 rows, 1.0 rounds 75 / 69, 250 rows, 2.3 rounds 199 / 186.
     auto fits = [&](int bm) { return q.block_m % bm == 0 || bm % q.block_m == 0; };
     // Less than three rounds count whole: blocks of 128 and more by what narrow tiles would take (of whose rounds what is left over runs
-    // beside the end of the one before), smaller ones by how full the rounds are - and around one round of few
-    // channels not at all, where wide tiles of 175 rows are 12 % ahead: how many tiles blocks put together make is known on the device
-    // only, and one more is a second round.
+    // beside the end of the one before), smaller ones by how full the rounds are.  Smaller blocks around one round (0.9 to 1.1) stay on
+    // narrow tiles: how many tiles they make is known on the device only, and one more is a second round.  64 x 128 / 128 x 256 there, us, even
+    // routing and then uneven (scores of the first expert two standard deviations above the last's), blocks of 64, groups of 128: 16 experts
+    // N=4096 K=4096, 80 rows 80 / 66 and 80 / 117; 16 experts N=2048, 200 rows 81 / 66 and 81 / 118; per-channel tables, 8 experts N=4096
+    // K=14336, 200 rows 207 / 179 and 210 / 289; 4 experts N=16384 K=5120, 96 rows 84 / 74 and 84 / 92.  Taken wide are only those whose
+    // experts nearly fill their tiles (the estimate, which counts a partial tile more for each, comes to two rounds: from 97 rows with
+    // 4 experts), which lose less: N=16384 K=5120, 100 rows 84 / 74 and 83 / 90; K=4096 with groups of 128 82 / 69 and 82 / 83.
     const double rounds = moe_rounds(q, p.N, 128, 256, 256), whole = ceil(rounds - 0.05);
     bool wide = mean > 60 && (rounds >= 3 || (q.block_m % 128 == 0 ? moe_rounds(q, p.N, 64, 128, 512) + 0.25 > 1.5 * whole
                                                                    : (rounds >= 1.1 || moe_tiles_estimate(q, 128) * (p.N / 256) >= 512) && whole < 1.34 * rounds));
