@@ -73,12 +73,15 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
     constexpr int NCL = 4 * NH;                 // consecutive channels per lane
     // int4 weights scaled in fp32: the activations are the first MFMA operand, so that a lane's sums are of one weight row (two
     // channels) and a slab's fold takes two scales and two zero points per lane instead of eight of each; the weights enter as
-    // u = v + 8, 0 .. 15.  16 rows a pass: over 85 calls of seven matrices 4.5 % less time; 32 rows a
-    // pass 7 % less with per-channel tables, but 3 to 5 % more with groups over K=8192 (34.5 -> 36.5), which stay as they were.
+    // u = v + 8, 0 .. 15.  16 rows a pass: over 85 calls of seven matrices 4.5 % less time; 32 rows a pass 7 % less with per-channel
+    // tables.  32 rows with groups stay as they were, for groups of 128 over the largest matrices (old / new form, captured graphs, us:
+    // N=28672 K=8192 35.9 / 36.5; N=22016 K=4096 and N=17920 K=5120 within 1 %); with it stay groups of 64, where the new one is ahead (41.1 /
+    // 39.2, 23.2 / 22.0, 27.7 / 26.1 over the same matrices), and the gathered form (8 experts N=28672 K=6144, 20 tokens in blocks of 64
+    // 400 / 384, 100 tokens 409 / 398).
     constexpr bool ROWS = WBITS == 4 && !REFQ && !(G128 && MB == 2);
     // ... and with 64 rows a pass the four waves of a K part, which multiply the same activations, sum up the rows of one block each
-    // and hand the sums on through LDS: read a slab later, so that no barrier is added (53.5 us with MFMAs against ones for every block
-    // in every wave, 49.8 with shared sums; with 32 rows a pass the exchange costs more than the four MFMAs that it saves)
+    // and hand the sums on through LDS: read a slab later, so that no barrier is added (what it gives: compute_rows_64 below; with 32
+    // rows a pass the exchange costs more than the four MFMAs that it saves)
     constexpr bool DIST = ROWS && GSUB == 1 && MB == 4 && RT == 4;
     constexpr float c_off = WBITS == 4 ? (ADT == FNN_F16 ? 1024.f + 8.f : 128.f + 8.f)
                                        : (ADT == FNN_F16 ? 1024.f + 128.f : 128.f);
@@ -356,8 +359,10 @@ __global__ __launch_bounds__(512) void gemm_wo_panel_kernel(const WoArgs p, cons
     };
     // ROWS, 64 rows a pass: one block of 16 activation rows at a time - its fragments are read while the block before is multiplied,
     // and its sums are folded while the next one is.  Both waves of a SIMD cross the same barrier, so that in the form above each of the
-    // three waits for the one before: K=8192, N=28672, groups of 128, 64 rows 52.3 -> 49.5 us; with 32 rows a pass it is the other way round,
-    // 33.8 and 36.4, with 16 they are level.
+    // three waits for the one before.  It pays with the shared sums only.  K=8192, N=28672, groups of 128, 64 rows, captured graphs on one
+    // box, us: 53.4 before (weights first, 136 + q), 52.6 in the form above, 53.2 in this one with MFMAs against ones for every block in
+    // every wave, 49.4 with shared sums; N=22016 K=4096 30.0, 29.9, 30.2, 28.6; per-channel tables 48.4, 47.8, 50.4, 46.1.  With 32 rows a
+    // pass it is the other way round, 33.8 and 36.4, with 16 they are level.
     auto compute_rows_64 = [&](const char* stage, const v4u w0, const v4u w1, const bool last, const auto& sv, const auto& zv,
                                float* sums_now, const float* before) {
         v4u B[2][2][2];
